@@ -29,8 +29,8 @@ CFLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-result", "-Wno-unused-value", "-Wno-unused-function",
 ]
-SOURCES = ["context.cpp", "ntt.hip", "poly_ops.hip", "keyswitch.hip", "encode.hip",
-           "keygen.hip", "capi.cpp"]
+SOURCES = ["moddown.hip", "ntt.hip", "convert.hip", "rescale.hip", "small_ring.hip",
+           "poly_ops.hip", "keyswitch.hip", "encode.hip", "keygen.hip", "context.cpp", "capi.cpp"]
 
 
 def _compile(src: str) -> tuple[str, int, str]:

@@ -197,8 +197,11 @@ Context::Context(uint32_t log_n_, const uint64_t* q, uint32_t num_q, const uint6
       float f = (float)want;
       while ((double)f > want) f = std::nextafter(f, 0.0f);
       mc.rq = f;
+      mc.one = 1;
     }
   }
+  lazy16 = true;
+  for (uint64_t m : mods) lazy16 = lazy16 && m >= (1ull << 33) && m < (1ull << 60);
   d_const = upload(hconst);
   d_tw_fwd = upload(fwd);
   d_tw_inv = upload(inv);

@@ -55,7 +55,7 @@ struct ModConst {
   uint64_t qinv;       // q^-1 mod 2^64 (redc_lazy)
   uint64_t neg_q8;     // 2^64 - 8q (lazy_sub at 8q; 0 when 8q >= 2^64)
   float rq;            // 2^32 / q (1 - 2^-20), rounded down (reduce_est)
-  uint32_t pad_;
+  uint32_t one;        // 1, as a value the compiler does not know (shoup_acc)
 };
 
 // x mod q for a 128-bit x = hi * 2^64 + lo (any hi): hi * (2^64 mod q) by
@@ -135,6 +135,7 @@ struct Context {
   std::vector<uint64_t> mods;        // L + K
   std::vector<uint64_t> psi;         // minimal primitive 2N-th roots
   std::vector<ModConst> hconst;
+  bool lazy16 = false;               // every modulus in [2^33, 2^60): LIM = 16 (modarith.hpp)
 
   // device tables
   ModConst* d_const = nullptr;       // [L+K]
@@ -344,6 +345,10 @@ void ntt_forward(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
                  uint32_t nlimb, LimbMap map);
 void ntt_inverse(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
                  uint32_t nlimb, LimbMap map);
+// The column pass alone of the two-pass transforms (N >= 2^13): the first
+// pass of a forward transform or the last, scaled one of an inverse.
+void ntt_cols(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
+              LimbMap map, bool inverse);
 // Forward NTT of npoly one-poly [nlimb][N] operands held in separate
 // allocations; `table` is a device array of their npoly base pointers.
 void ntt_forward_table(Context& c, uint64_t* const* table, uint32_t npoly, uint32_t nlimb);
@@ -362,6 +367,11 @@ void ntt_inverse_ksk(Context& c, uint64_t* ext_p, uint32_t npoly, const ModDownE
 // for the inverse column stages + conversion P -> Q_l + forward column
 // stages (into y, blocked), and the last forward pass with the epilogue.
 bool moddown_fused_ok(const Context& c, uint32_t nq);
+// Its middle kernel, and whether that kernel takes these moduli and this
+// many conversion sources.
+bool convert_mid_ok(const Context& c, uint32_t nq, uint32_t nsrc);
+void moddown_mid(Context& c, const uint64_t* ext_p, uint64_t* y, uint32_t npoly, uint32_t nq,
+                 const ConvPlan& pl);
 void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uint32_t nq,
                    const ConvPlan& pl, const ModDownEpi& epi);
 // Rescale of [npoly][nq][N] into out [npoly][nq-1][N] (out != a) in four
@@ -381,6 +391,20 @@ void rescale_fused_many(Context& c, uint64_t* const* outs, const uint64_t* const
 bool modup_fused_ok(const Context& c, uint32_t nq, uint32_t count);
 void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
                  uint64_t* digits);
+// Rings of at most 2^12 (small_ring.hip).  ModUp in two launches and ModDown's
+// conversion inside its last one, where the conversions have at most 8
+// sources; its first pass (`_ksk`) and last pass alone; rescale in two.
+bool small_modup_ok(const Context& c, uint32_t nq);
+bool small_moddown_ok(const Context& c);
+void small_modup(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
+                 uint64_t* digits);
+void small_ring_ksk(Context& c, uint64_t* ext_p, uint32_t npoly, const ModDownEpi& epi);
+void small_ring_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq,
+                        const ModDownEpi& epi);
+void small_ring_moddown_conv(Context& c, const uint64_t* ext_p, uint32_t npoly, uint32_t nq,
+                             const ConvPlan& pl, const ModDownEpi& epi);
+void small_rescale(Context& c, uint64_t* const* outs, const uint64_t* const* as, uint32_t count,
+                   uint32_t npoly, uint32_t nq);
 // Forward NTT of the converted limbs of the ModUp digits of `count`
 // ciphertexts, [count][nd][nq+K][N].
 void ntt_forward_digits(Context& c, uint64_t* digits, uint32_t count, uint32_t nd, uint32_t nq);

@@ -39,21 +39,53 @@ FHE_HD uint64_t shoup_lazy4(uint64_t a, uint64_t w, uint64_t wp, uint64_t q) {
   return a * w - qt * q;
 }
 
-// shoup_lazy4 with the remainder accumulated against qneg = 2^64 - q:
-// a*w - qt*q = a*w + qt*qneg (mod 2^64), which the VALU forms with
-// v_mad_u64_u32 accumulations and no borrow chain.  Same quotient, so the
-// same value in [0, 4q).
-FHE_HD uint64_t shoup_lazy4n(uint64_t a, uint64_t w, uint64_t wp, uint64_t qneg) {
+// Keeps a value in vector registers in the form it has here.  The compiler
+// narrows a 64-bit sum of products whose low word alone is used to separate
+// 32-bit multiplies and adds; gfx950 issues v_mad_u64_u32 at the rate of
+// v_mul_lo_u32, so the wide form saves the adds.
+FHE_HD uint64_t keep64(uint64_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+v"(v));
+#endif
+  return v;
+}
+FHE_HD uint32_t keep32(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+v"(v));
+#endif
+  return v;
+}
+
+// x + T mod 2^64, T = a*w mod q plus 0..3 q in [0, 4q) for any a < 2^64:
+// shoup_lazy4's quotient, the remainder accumulated against qneg = 2^64 - q
+// (a*w - qt*q = a*w + qt*qneg mod 2^64).  Both the addend x and the four
+// products of the high word ride in v_mad_u64_u32 accumulations: 11 VALU
+// instructions with no borrow chain (measured in registers, the forward
+// butterfly built on it takes 16.7 issue cycles against 20.5 for adding x to
+// a finished product with 32-bit multiplies in the high word).  `one` is 1,
+// read from memory where it matters: v_mad_u64_u32(h, one, x) adds a 32-bit h
+// to a 64-bit x without first zero-extending it into a register pair.
+FHE_HD uint64_t shoup_acc(uint64_t x, uint64_t a, uint64_t w, uint64_t wp, uint64_t qneg,
+                           uint32_t one = 1) {
   const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
   const uint32_t p0 = (uint32_t)wp, p1 = (uint32_t)(wp >> 32);
   const uint32_t w0 = (uint32_t)w, w1 = (uint32_t)(w >> 32);
   const uint32_t n0 = (uint32_t)qneg, n1 = (uint32_t)(qneg >> 32);
   const uint64_t qt = (uint64_t)a1 * p1 + (((uint64_t)a0 * p1) >> 32) +
-                      (((uint64_t)a1 * p0) >> 32);
+                      (uint64_t)(uint32_t)(((uint64_t)a1 * p0) >> 32) * one;
   const uint32_t t0 = (uint32_t)qt, t1 = (uint32_t)(qt >> 32);
-  const uint64_t lo = (uint64_t)t0 * n0 + (uint64_t)a0 * w0;
-  const uint32_t hi = (uint32_t)(lo >> 32) + a0 * w1 + a1 * w0 + t0 * n1 + t1 * n0;
+  uint64_t lo = keep64(x + (uint64_t)a0 * w0);
+  lo += (uint64_t)t0 * n0;
+  uint64_t h = (uint64_t)a0 * w1 + (uint64_t)a1 * w0;
+  h += (uint64_t)t0 * n1;
+  h += (uint64_t)t1 * n0;
+  const uint32_t hi = keep32((uint32_t)(lo >> 32) + (uint32_t)keep64(h));
   return ((uint64_t)hi << 32) | (uint32_t)lo;
+}
+
+// a*w mod q plus 0..3 q, in [0, 4q) for any a < 2^64.
+FHE_HD uint64_t shoup_lazy4n(uint64_t a, uint64_t w, uint64_t wp, uint64_t qneg) {
+  return shoup_acc(0, a, w, wp, qneg);
 }
 
 // x >= m ? x - m : x for nm = 2^64 - m, m <= 2^63 and x - m < 2^63 when
@@ -128,6 +160,62 @@ FHE_HD uint64_t reduce_est(uint64_t x, uint64_t qneg, float rq) {
   const uint64_t r = x + (uint64_t)e * qneg;
   const uint64_t d = r + qneg;
   return (int64_t)d < 0 ? r : d;
+}
+
+// ---- NTT butterflies on lazy ranges ----
+// Values are kept below LIM q: LIM = 16 for moduli in [2^33, 2^60) (16q <
+// 2^64; reduce_est's range), 8 for any q < 2^61.  Where a sum would pass the
+// limit its operand is first brought below LIM/2 q by one conditional
+// subtraction; which stages need that follows from the bounds alone, so it
+// is decided at compile time (fwd_reduces, and the bounds inv_butterfly
+// tracks): a forward pass reduces on 3 or 4 of 8 stages, an inverse one on
+// about 60% of its sums.
+struct LazyMod {
+  uint64_t q4, q8, neg_q, neg_half;  // neg_half = 2^64 - (LIM/2) q
+  uint32_t one;                      // 1 (shoup_acc)
+};
+
+// Forward (Cooley-Tukey): (x + y w, x - y w + 4q) with x first brought below
+// LIM/2 q when `red`; both outputs are below (bound of x) + 4q, y is any word.
+FHE_HD void fwd_butterfly(uint64_t& x, uint64_t& y, uint64_t w, uint64_t wp, const LazyMod& m,
+                          bool red) {
+  const uint64_t X = red ? lazy_sub(x, m.neg_half) : x;
+  x = shoup_acc(X, y, w, wp, m.neg_q, m.one);
+  y = (X << 1) + m.q4 - x;
+}
+// Whether forward stage `beta` of a pass (stages S-1 .. 0, named by the index
+// bit they pair) reduces its x, given x below b q.  LIM = 16: only on even
+// beta, and only if this stage and the next could pass the limit; so every
+// pass whose input is below 12q leaves values below 12q, which the next pass
+// and the ModDown epilogue (another 3q on top) accept.  LIM = 8: whenever
+// this stage could pass it, leaving values below 8q.
+constexpr bool fwd_reduces_at(int lim, int b, int beta) {
+  return lim == 16 ? beta % 2 == 0 && b + 8 > 16 : b + 4 > lim;
+}
+// Bound (in q) of the values entering stage `beta` of a pass of S stages
+// whose input is below b q (beta = -1: the pass's output).
+constexpr int fwd_bound(int lim, int b, int S, int beta) {
+  for (int k = S - 1; k > beta; --k) b = (fwd_reduces_at(lim, b, k) ? lim / 2 : b) + 4;
+  return b;
+}
+constexpr bool fwd_reduces(int lim, int b, int S, int beta) {
+  return fwd_reduces_at(lim, fwd_bound(lim, b, S, beta), beta);
+}
+// The bound every forward pass leaves.
+constexpr int fwd_pass_bound(int lim) { return lim == 16 ? 12 : 8; }
+
+// Inverse (Gentleman-Sande): (x + y, (x - y) w).  bx and by are the bounds
+// (in q) of x and y on entry and of the two outputs on return: the sum is
+// reduced only where it may reach LIM/2 q, the product is below 4q.
+FHE_HD void inv_butterfly(uint64_t& x, uint64_t& y, uint64_t w, uint64_t wp, const LazyMod& m,
+                          int lim, int& bx, int& by) {
+  const uint64_t s = x + y;
+  const uint64_t d = x + (by <= 4 ? m.q4 : m.q8) - y;
+  y = shoup_acc(0, d, w, wp, m.neg_q, m.one);
+  const bool red = bx + by > lim / 2;
+  x = red ? lazy_sub(s, m.neg_half) : s;
+  bx = red ? lim / 2 : bx + by;
+  by = 4;
 }
 
 // 128-bit accumulator for sums of products that are reduced once.
