@@ -276,6 +276,10 @@ void modup_batch(Context& c, const uint64_t* const* as, uint32_t count, uint32_t
     modup_fused(c, as, count, nq, digits);
     return;
   }
+  if (small_modup_ok(c, nq)) {
+    small_modup(c, as, count, nq, digits);
+    return;
+  }
   const size_t n = c.n, ne = nq + c.K, pl = (size_t)nq * n;
   const uint32_t nd = num_digits(c, nq);
   const size_t ct_words = (size_t)nd * ne * n;
@@ -370,7 +374,8 @@ void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
   const size_t n = c.n, ne = nq + c.K, kw = (size_t)c.K * n;
   // The fused Q-limb products are reduced once: nd * q_i < 2^64 holds for
   // nd <= 8 and q_i < 2^61.
-  Scratch ext(c, 2 * (size_t)batch * kw), y(c, 2 * (size_t)batch * nq * n);
+  const bool small = small_moddown_ok(c);  // no y: converted as the last pass loads
+  Scratch ext(c, 2 * (size_t)batch * kw), y(c, small ? 1 : 2 * (size_t)batch * nq * n);
   ModDownEpi epi{};
   epi.mc = c.d_const;
   epi.kl = (size_t)(c.L + c.K) * n;
@@ -394,6 +399,10 @@ void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
     return;
   }
   ntt_inverse_ksk(c, ext.p, 2 * batch, epi);
+  if (small) {
+    small_ring_moddown_conv(c, ext.p, 2 * batch, nq, c.moddown_plan(nq), epi);
+    return;
+  }
   convert(c, c.moddown_plan(nq), ext.p, kw, y.p, (size_t)nq * n, nq, 2 * batch);
   ntt_forward_moddown(c, y.p, 2 * batch, nq, epi);
 }

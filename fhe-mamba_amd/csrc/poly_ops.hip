@@ -304,26 +304,6 @@ __global__ void __launch_bounds__(TPB)
   }
 }
 
-// Rescale step 1: centred lift of the (inverse-NTT'd) last limb into limbs
-// i < l.  grid (N/512, l, npoly).  last: [npoly][N] coefficient form.
-__global__ void __launch_bounds__(TPB)
-    k_rescale_lift(uint64_t* t, const uint64_t* last, const ModConst* mc, const uint64_t* rs,
-                   uint32_t n, uint32_t l, uint32_t L, uint64_t ql) {
-  const uint32_t i = blockIdx.y;
-  const uint64_t q = mc[i].q;
-  const uint64_t qlm = rs[((size_t)l * L + i) * 4];  // q_l mod q_i
-  const size_t e = pair_off();
-  const U2 v = ld2(last + (size_t)blockIdx.z * n + e);
-  const uint64_t half = ql >> 1;
-  const ModConst m = mc[i];
-  auto lift = [&](uint64_t x) -> uint64_t {
-    // x mod q_i (x < 2^61 may exceed q_i), minus q_l if x is in the upper half.
-    const uint64_t r = reduce_2q(x - mulhi64(x, m.mu64) * q, q);
-    return x > half ? sub_mod(r, qlm, q) : r;
-  };
-  st2(t + ((size_t)blockIdx.z * l + i) * n + e, lift(v.x), lift(v.y));
-}
-
 // ModRaise lift: x [npoly][N] in coefficient form mod q0 -> out[p][j] =
 // (x centred mod q0) mod q_j for j < nq.  grid (N/512, nq, npoly).
 __global__ void __launch_bounds__(TPB)
@@ -341,20 +321,6 @@ __global__ void __launch_bounds__(TPB)
     return a > half ? sub_mod(r, q0m, q) : r;
   };
   st2(out + ((size_t)blockIdx.z * nq + j) * n + e, lift(v.x), lift(v.y));
-}
-
-// Rescale step 2: out_i = (a_i - t_i) * q_l^-1.  grid (N/512, l, npoly).
-__global__ void __launch_bounds__(TPB)
-    k_rescale_combine(uint64_t* out, const uint64_t* a, const uint64_t* t, const ModConst* mc,
-                      const uint64_t* rs, uint32_t n, uint32_t l, uint32_t L) {
-  const uint32_t i = blockIdx.y;
-  const uint64_t q = mc[i].q;
-  const uint64_t inv = rs[((size_t)l * L + i) * 4 + 1], invs = rs[((size_t)l * L + i) * 4 + 2];
-  const size_t e = pair_off();
-  const U2 x = ld2(a + ((size_t)blockIdx.z * (l + 1) + i) * n + e);
-  const U2 y = ld2(t + ((size_t)blockIdx.z * l + i) * n + e);
-  st2(out + ((size_t)blockIdx.z * l + i) * n + e, shoup(x.x + q - y.x, inv, invs, q),
-      shoup(x.y + q - y.y, inv, invs, q));
 }
 
 LimbConsts make_consts(const Context& c, const uint64_t* consts, uint32_t nlimb) {
@@ -548,14 +514,7 @@ void poly_rescale(Context& c, uint64_t* out, const uint64_t* a, uint32_t npoly, 
     rescale_fused(c, out, a, npoly, nq);
     return;
   }
-  const uint32_t l = nq - 1;
-  Scratch last(c, (size_t)npoly * c.n), t(c, (size_t)npoly * l * c.n);
-  // last limb of every poly -> [npoly][N], to coefficient form with q_l
-  FHE_LAUNCH(c, "k_copy_limbs", k_copy_limbs, grid_for(c, 1, npoly), dim3(tpb_for(c)), 0, last.p, 1u, a + (size_t)l * c.n, nq, c.n);
-  ntt_inverse(c, last.p, npoly, c.n, 1, LimbMap::contiguous(l));
-  FHE_LAUNCH(c, "k_rescale_lift", k_rescale_lift, grid_for(c, l, npoly), dim3(tpb_for(c)), 0, t.p, last.p, c.d_const, c.d_rescale, c.n, l, c.L, c.mods[l]);
-  ntt_forward(c, t.p, npoly, (size_t)l * c.n, l, LimbMap::contiguous(0));
-  FHE_LAUNCH(c, "k_rescale_combine", k_rescale_combine, grid_for(c, l, npoly), dim3(tpb_for(c)), 0, out, a, t.p, c.d_const, c.d_rescale, c.n, l, c.L);
+  small_rescale(c, &out, &a, 1, npoly, nq);
 }
 
 void poly_rescale_many(Context& c, uint64_t* const* outs, const uint64_t* const* as,
@@ -565,7 +524,7 @@ void poly_rescale_many(Context& c, uint64_t* const* outs, const uint64_t* const*
     rescale_fused_many(c, outs, as, count, npoly, nq);
     return;
   }
-  for (uint32_t r = 0; r < count; ++r) poly_rescale(c, outs[r], as[r], npoly, nq);
+  small_rescale(c, outs, as, count, npoly, nq);
 }
 
 
