@@ -282,7 +282,7 @@ Context::~Context() {
     hipFree(pl->d_qhat_inv);
     hipFree(pl->d_src_scale);
     hipFree(pl->d_qhat_mont);
-    hipFree(pl->d_qhat_mont30);
+    hipFree(pl->d_bytes);
     hipFree(pl->d_dst_idx);
     hipFree(pl->d_src_idx32);
   }
@@ -310,7 +310,7 @@ ConvPlan* Context::build_plan(const std::vector<uint32_t>& src, const std::vecto
   pl->src_idx = src;
   pl->dst_idx = dst;
   std::vector<uint64_t> qhat_inv(2 * src.size()), qhat_mont(src.size() * dst.size());
-  std::vector<uint64_t> qhat_mont30(src.size() * dst.size());
+  std::vector<uint64_t> qhat(src.size() * dst.size());
   std::vector<uint64_t> src_scale(2 * src.size());
   for (size_t a = 0; a < src.size(); ++a) {
     const uint64_t qa = mods[src[a]];
@@ -330,13 +330,38 @@ ConvPlan* Context::build_plan(const std::vector<uint32_t>& src, const std::vecto
         if (b != a) hk = host_mulmod(hk, mods[src[b]] % t, t);
       if (factor) hk = host_mulmod(hk, (*factor)[k] % t, t);
       qhat_mont[a * dst.size() + k] = host_to_mont(hk, t);
-      qhat_mont30[a * dst.size() + k] =
-          host_mulmod(qhat_mont[a * dst.size() + k], (1ull << 30) % t, t);
+      qhat[a * dst.size() + k] = hk;
     }
   }
   pl->d_qhat_inv = upload(qhat_inv);
   pl->d_qhat_mont = upload(qhat_mont);
-  pl->d_qhat_mont30 = upload(qhat_mont30);
+  if (src.size() <= 16) {
+    // Operand rows: lane l holds row l % 32 and sources 4 ks + 2 (l / 32) +
+    // {0, 1}.  A lane of the result holds rows 4 (l / 32) + {0..3} + 8 {0..3},
+    // so row r carries sum o = (r & 3) + 4 (r >> 3) of that lane: byte o % 8 of target
+    // 2 ((r >> 2) & 1) + o / 8 of the group: each half of the wavefront
+    // gets all eight sums of two targets.
+    const size_t groups = (dst.size() + 3) / 4, ksteps = (src.size() + 3) / 4;
+    std::vector<int8_t> bytes(groups * ksteps * 64 * 16, 0);
+    for (size_t i = 0; i < src.size(); ++i)
+      for (size_t k = 0; k < dst.size(); ++k) {
+        const uint64_t t = mods[dst[k]];
+        uint64_t v = host_mulmod(qhat[i * dst.size() + k], (1ull << 32) % t, t);
+        const uint32_t j = k % 4, lane_hi = (i % 4) / 2;
+        for (uint32_t a = 0; a < 8; ++a) {
+          const uint64_t bal = v + 0x8080808080808080ull;  // byte b + 128 in byte b
+          for (uint32_t b = 0; b < 8; ++b) {
+            const uint32_t o = 8 * (j & 1) + b;  // index among the lane's 16 rows
+            const uint32_t r = (o & 3) + 8 * (o >> 2) + 4 * (j >> 1);
+            const size_t lane = r + 32 * lane_hi;
+            bytes[(((k / 4) * ksteps + i / 4) * 64 + lane) * 16 + 8 * (i % 2) + a] =
+                (int8_t)(uint8_t)((bal >> (8 * b)) ^ 0x80);
+          }
+          v = host_mulmod(v, 256 % t, t);
+        }
+      }
+    pl->d_bytes = upload(bytes);
+  }
   pl->d_src_scale = upload(src_scale);
   pl->d_dst_idx = upload(dst);
   pl->d_src_idx32 = upload(src);

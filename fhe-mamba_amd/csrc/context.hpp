@@ -83,7 +83,11 @@ struct ConvPlan {
   // inverse NTT's scaling folded in, for conversions fused after a transform.
   uint64_t* d_src_scale = nullptr;         // [nsrc][2]
   uint64_t* d_qhat_mont = nullptr;         // [nsrc][ndst]
-  uint64_t* d_qhat_mont30 = nullptr;       // [nsrc][ndst]: qhat_mont * 2^30 mod t_k
+  // The constants for the matrix units: balanced bytes of
+  // [Qhat_i * 2^8a * 2^32]_{t_k} for a = 0..7, [ceil(ndst / 4)][ceil(nsrc / 4)]
+  // [64 lanes][16 bytes] in the operand layout of v_mfma_i32_32x32x32_i8
+  // (build_plan); absent above 16 sources.
+  int8_t* d_bytes = nullptr;
   uint32_t* d_dst_idx = nullptr;           // [ndst]
   uint32_t* d_src_idx32 = nullptr;         // [nsrc]
 };

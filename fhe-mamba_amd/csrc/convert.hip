@@ -1,4 +1,5 @@
 // The conversion middle kernel of ModUp and ModDown, and ModUp's own passes.
+
 #include "ntt_body.hpp"
 
 namespace fhe {
@@ -28,27 +29,34 @@ __global__ void __launch_bounds__(256)
       digits, poly_stride, mc, tw_all, log_n, map, s_other, 1, PlainStore{});
 }
 
-// ---- Fused middle of a batched ModDown, ring dimensions 2^13 .. 2^17 ----
+// ---- Fused middle of ModUp and of a batched ModDown, N = 2^13 .. 2^17 ----
 //
-// One workgroup per (poly, column u): the last S1 inverse stages of the K
-// P limbs (the column stages; the first pass wrote the blocked P limbs), the
-// scaling by N^-1 * [P/p_t]^-1 folded into one Shoup product, the fast
-// conversion P -> Q_l (30-bit split MACs, one REDC per output, constants in
-// Montgomery form with -P^-1 folded in), and the first S1 forward stages of
-// every Q limb, written to the blocked y.  This replaces an inverse column
-// pass, a conversion and a forward column pass, and the three round trips
-// of the P limbs and y through HBM between them.
+// One workgroup per (poly, column u): the last S1 inverse stages of the
+// source limbs (the column stages; the first pass wrote them in the blocked
+// layout), the scaling by N^-1 * [Q/q_t]^-1 folded into one Shoup product, the
+// fast basis conversion, and the first S1 forward stages of every target
+// limb, written blocked.  This replaces an inverse column pass, a conversion
+// and a forward column pass, and the round trips through HBM between them.
 //
 // Each column line of M = 2^S1 rows belongs to TPL = min(64, M / 4) lanes of
 // one wavefront (radix M / TPL per lane), so its sub-passes exchange through
-// LDS with wavefront-level ordering only; the four waves of a workgroup meet
-// at a single barrier, once the converted sources are in LDS.  With one line
-// per wave the modulus, its twiddles and the conversion constants are
-// wavefront-uniform.  Stage order, twiddle indices and lazy ranges are those
-// of the column passes of ntt_body.  Workgroups have NW waves: 4 for large
-// batches, 8 when a launch has too few (poly, column) tiles to fill the
-// chip, which halves each workgroup's serial line count and doubles the
-// waves in flight.
+// LDS with wavefront-level ordering only.  With one line per wave the modulus
+// and its constants are wavefront-uniform.  Targets go in batches of one line
+// per line in flight: the workgroup converts a batch into the lines, meets,
+// and each wavefront transforms its own.
+//
+// The conversion y_k = sum_i v_i c_ik mod t_k is a contraction over the
+// sources, done on the int8 matrix units.  v_i is held as eight balanced bytes
+// s_ia (v = sum_a s_ia 2^8a, s in [-128, 127]), and the table holds the
+// balanced bytes of C_iak = c_ik 2^8a 2^32 mod t_k, so
+//   T_k = sum_ia s_ia C_iak = sum_b 2^8b S_kb,   S_kb = sum_ia s_ia byte_b(C_iak)
+// with |S_kb| <= 8 K 2^14 <= 2^21 exact in 32 bits: v_mfma_i32_32x32x32_i8
+// gives the eight sums of four targets (32 rows) at 32 column rows (32
+// columns) from four sources a step.  One 32-bit Montgomery step of the about
+// 75-bit T_k, T_k + m t_k = 2^32 r, leaves r = sum_i v_i c_ik in (0, 3 t_k)
+// after adding t_k.  Per output that is about 17 VALU instructions whatever
+// the number of sources, where 64-bit multiply-adds took 4 a source and 25.
+constexpr uint32_t MAX_CONV_SRC = 16;
 
 template <int S1>
 constexpr uint32_t mid_pitch() {
@@ -57,10 +65,6 @@ constexpr uint32_t mid_pitch() {
 template <int S1>
 constexpr int mid_lanes_per_line() {
   return (1 << S1) / 4 < 64 ? (1 << S1) / 4 : 64;
-}
-template <int S1, int NW>
-constexpr int mid_lines() {  // lines in flight per workgroup of NW waves
-  return NW * (64 / mid_lanes_per_line<S1>());
 }
 
 // What one (poly, column) tile converts.  Poly p of the launch uses plan
@@ -76,8 +80,7 @@ constexpr int mid_lines() {  // lines in flight per workgroup of NW waves
 constexpr int MID_MAXPLAN = 8;
 struct MidPlan {
   const uint64_t* src_scale;  // [nsrc][2]: [Q/q_t]^-1 N^-1 mod q_t (Shoup)
-  const uint64_t* qhat_mont;  // [nsrc][ndst], Montgomery form w.r.t. the target
-  const uint64_t* qhat_mont30;  // [nsrc][ndst], qhat_mont * 2^30 mod the target
+  const int8_t* bytes;        // ConvPlan::d_bytes
   uint32_t nsrc, ndst, src_mod0, src_limb0, skip_at, skip_len, qlimbs;
 };
 struct MidArgs {
@@ -88,248 +91,252 @@ struct MidArgs {
   uint32_t nplan, L;
 };
 
-// One group of at most eight conversion sources i0 .. i1 - 1 for target k:
-// T_g = t + u 2^64 == sum_i v_i c_ik (mod t_k), from sources held as 30-bit
-// halves (vl, vh) and the Montgomery-form tables c and c' = c 2^30 mod t_k
-// split into 30-bit halves: v c == vl c + vh c', so b0 = sum vl cl + vh dl
-// and b1 = sum vl ch + vh dh (each below 16 2^60 = 2^64) give T_g = b0 +
-// b1 2^30, whose high word u is at most 2^30.
-template <int R, uint32_t VSTEP, uint32_t PITCH, class CU64>
-__device__ __forceinline__ void conv_group(const uint64_t* sbase, CU64* qhat_mont,
-                                           CU64* qhat_mont30, uint32_t nq, uint32_t k,
-                                           uint32_t i0, uint32_t i1, uint64_t (&t)[R],
-                                           uint64_t (&u)[R]) {
-  constexpr uint32_t M30 = (1u << 30) - 1;
-  uint64_t b0[R], b1[R];
-#pragma unroll
-  for (int v = 0; v < R; ++v) b0[v] = b1[v] = 0;
-  for (uint32_t i = i0; i < i1; ++i) {
-    const uint64_t cv = qhat_mont[(size_t)i * nq + k];
-    const uint64_t dv = qhat_mont30[(size_t)i * nq + k];
-    const uint64_t* sl = sbase + (size_t)i * PITCH;
-    uint64_t sv[R];
-#pragma unroll
-    for (int v = 0; v < R; ++v) sv[v] = sl[v * VSTEP];
-    // the constants' and all R elements' reads in flight before the first
-    // product: one wait a source
-    __builtin_amdgcn_sched_barrier(0);
-    const uint32_t cl = (uint32_t)cv & M30, ch = (uint32_t)(cv >> 30);
-    const uint32_t dl = (uint32_t)dv & M30, dh = (uint32_t)(dv >> 30);
-#pragma unroll
-    for (int v = 0; v < R; ++v) {
-      const uint32_t vl = (uint32_t)sv[v], vh = (uint32_t)(sv[v] >> 32);
-      b0[v] += (uint64_t)vl * cl + (uint64_t)vh * dl;
-      b1[v] += (uint64_t)vl * ch + (uint64_t)vh * dh;
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < R; ++v) {
-    const uint64_t m = b1[v] << 30;
-    t[v] = b0[v] + m;
-    u[v] = (b1[v] >> 34) + (t[v] < m);
-  }
-}
+// Target constants of the conversion, in LDS.
+struct MidTarget {
+  uint64_t q;
+  uint32_t qinv_neg;  // -q^-1 mod 2^32
+  uint32_t pad_;
+};
 
-// Body for (poly, column) tile `tile` with (K + NL) PITCH words of lds.
-template <int S1, int S2, int NW>
+// Body for (poly, column) tile `tile` of a workgroup of nw waves (a multiple
+// of 4), with mid_lds_bytes of lds.
+template <int S1, int S2>
 __device__ __forceinline__ void convert_mid_body(const MidArgs& a, const ModConst* __restrict__ mc,
                                                  const uint64_t* __restrict__ tw_inv,
                                                  const uint64_t* __restrict__ tw_fwd,
-                                                 uint32_t tile, uint64_t* lds_dyn) {
+                                                 uint32_t tile, uint32_t nw, uint64_t* lds_dyn) {
   constexpr int M = 1 << S1, TPL = mid_lanes_per_line<S1>(), R = M / TPL;
-  constexpr int RHO = R == 4 ? 2 : 3, LPW = 64 / TPL, NL = mid_lines<S1, NW>();
+  constexpr int RHO = R == 4 ? 2 : 3, LPW = 64 / TPL;
   constexpr int NSP = (S1 + RHO - 1) / RHO;
   constexpr uint32_t PITCH = mid_pitch<S1>(), N2 = 1u << S2;
   constexpr size_t N = (size_t)M << S2;
-  constexpr uint32_t M30 = (1u << 30) - 1;
   static_assert(R * TPL == M && (1 << RHO) == R, "column split");
+  const uint32_t nl = nw * LPW;
   const uint32_t p = tile / N2, col = tile % N2;
   const MidPlan& pl = a.plan[p % a.nplan];
   const uint32_t K = pl.nsrc, nq = pl.ndst;
   const uint64_t* const ext = a.src + (size_t)(p / a.nplan) * a.src_group_words +
                               (size_t)pl.src_limb0 * N;
   uint64_t* const y = a.out + (size_t)p * a.out_group_words;
-  // The conversion tables are read-only for the whole launch: reading them
-  // through the constant address space lets uniform loads use the scalar
-  // cache, as for kernel-argument tables.
+  // The tables are read-only for the whole launch: reading them through the
+  // constant address space lets uniform loads use the scalar cache, as for
+  // kernel-argument tables.
   typedef const uint64_t __attribute__((address_space(4))) cu64;
   cu64* const src_scale = (cu64*)pl.src_scale;
-  cu64* const qhat_mont = (cu64*)pl.qhat_mont;
-  cu64* const qhat_mont30 = (cu64*)pl.qhat_mont30;
-  uint64_t* const src = lds_dyn;
-  uint64_t* const work = lds_dyn + (size_t)K * PITCH;
+  const uint32_t groups = (nq + 3) / 4;  // of four targets
+  MidTarget* const tgt = reinterpret_cast<MidTarget*>(lds_dyn);
+  uint64_t* const src = lds_dyn + (size_t)groups * 4 * (sizeof(MidTarget) / 8);
+  uint64_t* const work = src + (size_t)K * PITCH;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63, sub = lane / TPL, tau = lane % TPL;
   const uint32_t first = wave * LPW + sub;
+  auto target_mod = [&](uint32_t k, uint32_t& kpos) {
+    kpos = k < pl.skip_at ? k : k + pl.skip_len;
+    return kpos < pl.qlimbs ? kpos : a.L + (kpos - pl.qlimbs);
+  };
 
-  // Inverse column stages of the P limbs; each limb is one line of src.
-  for (uint32_t t = first; t < K; t += NL) {
+  for (uint32_t k = threadIdx.x; k < 4 * groups; k += 64 * nw) {
+    uint32_t kpos;
+    const uint32_t m = target_mod(k < nq ? k : nq - 1, kpos);
+    tgt[k] = MidTarget{mc[m].q, (uint32_t)mc[m].qinv_neg, 0};
+  }
+
+  // Inverse column stages of the source limbs; each limb is one line of src.
+  for (uint32_t t = first; t < K; t += nl) {
     const uint32_t midx = pl.src_mod0 + t;
     const uint64_t q = mc[midx].q;
     const LazyMod lm = lazy_mod<16>(mc[midx]);
     const uint64_t* __restrict__ tw = tw_inv + (size_t)midx * N * 2;
     uint64_t* const line = src + (size_t)t * PITCH;
-    uint64_t x[R];
+    uint64_t x[R], twx[2][R - 1], twy[2][R - 1];
     int bnd[R];  // bounds of x in q
     // First window (bits 0 .. RHO-1): rows R tau + v, one blocked run.
     const uint64_t* g = ext + (size_t)t * N + blocked_off<S2>(R * tau, col);
 #pragma unroll
     for (int v = 0; v < R; ++v) x[v] = g[v];
-#pragma unroll
-    for (int sp = 0; sp < NSP; ++sp) {
-      const int lo = RHO * sp;
-      const int w = lo + RHO <= S1 ? lo : S1 - RHO;
-      const int bhi = lo + RHO <= S1 ? lo + RHO - 1 : S1 - 1;
+    fetch_twiddles<S1, RHO, true, 0, LPW == 1>(tw, 1, tau, twx[0], twy[0]);
+    static_for<NSP>([&](auto spc) {
+      constexpr int sp = decltype(spc)::value;
+      using W = SubPass<S1, RHO, true, sp>;
+      constexpr int w = W::w;
       const uint32_t thi = (tau >> w) << (w + RHO), tlo = tau & ((1u << w) - 1);
       if (sp > 0) {
 #pragma unroll
         for (int v = 0; v < R; ++v) x[v] = line[lds_idx(0, thi | ((uint32_t)v << w) | tlo, 0)];
       }
+      if constexpr (sp + 1 < NSP)
+        fetch_twiddles<S1, RHO, true, sp + 1, LPW == 1>(tw, 1, tau, twx[(sp + 1) & 1],
+                                                        twy[(sp + 1) & 1]);
 #pragma unroll
       for (int v = 0; v < R; ++v) bnd[v] = 8;
 #pragma unroll
-      for (int beta = lo; beta <= bhi; ++beta) {
-        const int d = 1 << (beta - w);
+      for (int k = 0; k < RHO; ++k) {
+        const int beta = w + k, d = 1 << k;
+        if (beta < W::blo || beta > W::bhi) continue;
 #pragma unroll
         for (int v = 0; v < R; ++v) {
           if (v & d) continue;
-          const uint32_t u = thi | ((uint32_t)v << w) | tlo;
-          const uint32_t ti = (1u << (S1 - 1 - beta)) | (u >> (beta + 1));
-          const uint64_t wv = tw[2 * ti], ws = tw[2 * ti + 1];
-          inv_butterfly(x[v], x[v + d], wv, ws, lm, 16, bnd[v], bnd[v + d]);
+          const int ti = twiddle_at<RHO>(k, v);
+          inv_butterfly(x[v], x[v + d], twx[sp & 1][ti], twy[sp & 1][ti], lm, 16, bnd[v],
+                        bnd[v + d]);
         }
       }
       if (sp == NSP - 1) {
-        // v_t = x N^-1 [P/p_t]^-1 mod p_t, stored as 30-bit halves.
+        // v_t = x N^-1 [Q/q_t]^-1 mod q_t as balanced bytes: adding 128 to
+        // every byte with carries leaves byte_a + 128 in byte a.
         const uint64_t f = src_scale[2 * t], fs = src_scale[2 * t + 1];
 #pragma unroll
         for (int v = 0; v < R; ++v) {
-          const uint64_t z = reduce_4q(shoup_lazy4(x[v], f, fs, q), q);
-          x[v] = ((uint64_t)(uint32_t)(z >> 30) << 32) | ((uint32_t)z & M30);
+          const uint64_t z = reduce_4q(shoup_acc(0, x[v], f, fs, lm.neg_q, lm.one), q);
+          x[v] = (z + 0x8080808080808080ull) ^ 0x8080808080808080ull;
         }
       }
       wave_lds_sync();
 #pragma unroll
       for (int v = 0; v < R; ++v) line[lds_idx(0, thi | ((uint32_t)v << w) | tlo, 0)] = x[v];
       wave_lds_sync();
-    }
+    });
   }
   __syncthreads();
 
-  // Conversion into the Q limbs, one line of `work` per line in flight, then
-  // their forward column stages.
+  // Batches of nl targets.  The conversion's work units are (four targets, 32
+  // rows); each wave takes UPW consecutive ones of one group of four targets.
+  constexpr uint32_t BLKS = M / 32, UPW = LPW * M / 128;
+  static_assert(UPW >= 1 && BLKS % UPW == 0, "conversion units");
+  typedef int v4i __attribute__((ext_vector_type(4)));
+  typedef int v16i __attribute__((ext_vector_type(16)));
+  typedef unsigned long long v2u __attribute__((ext_vector_type(2)));
+  const uint32_t ksteps = (K + 3) / 4, half = lane >> 5, col32 = lane & 31;
+  const uint32_t ugrp = wave * UPW / BLKS, ublk = wave * UPW % BLKS;
   uint64_t* const line = work + (size_t)first * PITCH;
-  for (uint32_t k = first; k < nq; k += NL) {
-    const uint32_t kpos = k < pl.skip_at ? k : k + pl.skip_len;
-    const uint32_t kmod = kpos < pl.qlimbs ? kpos : a.L + (kpos - pl.qlimbs);
-    const uint64_t q = mc[kmod].q, qn = mc[kmod].qinv;
+  for (uint32_t k0 = 0; k0 < nq; k0 += nl) {
+    const uint32_t tg = k0 / 4 + ugrp;
+    if (tg < groups) {
+      const v4i* const tab = reinterpret_cast<const v4i*>(pl.bytes) + (size_t)tg * ksteps * 64 + lane;
+      MidTarget mt[2];
+#pragma unroll
+      for (int o = 0; o < 2; ++o) mt[o] = tgt[4 * tg + 2 * half + o];
+#pragma unroll
+      for (uint32_t u = 0; u < UPW; ++u) {
+        const uint32_t row = 32 * (ublk + u) + col32;
+        const uint64_t* const sp = src + lds_idx(0, row, 0);
+        v16i acc = {};
+        for (uint32_t ks = 0; ks < ksteps; ++ks) {
+          const v4i ab = tab[ks * 64];
+          // sources past K meet zero table bytes; any line will do for them
+          const uint32_t i0 = 4 * ks + 2 * half, i1 = i0 + 1;
+          v2u sv;
+          sv.x = sp[(size_t)(i0 < K ? i0 : K - 1) * PITCH];
+          sv.y = sp[(size_t)(i1 < K ? i1 : K - 1) * PITCH];
+          acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ab, __builtin_bit_cast(v4i, sv), acc, 0, 0,
+                                                      0);
+        }
+#pragma unroll
+        for (int o = 0; o < 2; ++o) {
+          const int p01 = acc[8 * o] + (acc[8 * o + 1] << 8);
+          const int p23 = acc[8 * o + 2] + (acc[8 * o + 3] << 8);
+          const int p45 = acc[8 * o + 4] + (acc[8 * o + 5] << 8);
+          const int p67 = acc[8 * o + 6] + (acc[8 * o + 7] << 8);
+          // T = L + 2^32 H;  r = (T + m q) / 2^32 + q
+          const int64_t L = (int64_t)p23 * 65536 + p01;
+          const int64_t H = (int64_t)p67 * 65536 + p45;
+          const uint32_t q0 = (uint32_t)mt[o].q, q1 = (uint32_t)(mt[o].q >> 32);
+          const uint32_t m = (uint32_t)L * mt[o].qinv_neg;
+          const uint64_t lo = (uint64_t)m * q0 + (uint32_t)L;  // low word 0
+          uint64_t r = mt[o].q + (uint64_t)H + (uint64_t)(L >> 32);
+          r += lo >> 32;
+          r += (uint64_t)m * q1;
+          work[(size_t)(4 * ugrp + 2 * half + o) * PITCH + lds_idx(0, row, 0)] = r;
+        }
+      }
+    }
+    const uint32_t k = k0 + first;
+    uint32_t kpos;
+    const uint32_t kmod = target_mod(k < nq ? k : nq - 1, kpos);
     const LazyMod lm = lazy_mod<16>(mc[kmod]);
     const uint64_t* __restrict__ tw = tw_fwd + (size_t)kmod * N * 2;
-    uint64_t x[R];
-    {
-      // First forward window (bits S1-RHO .. S1-1): rows thi | v << w | tlo.
-      constexpr int w = S1 - RHO;
-      // With w >= 4 the row fields do not interact with the u / 16 padding:
-      // lds_idx(thi | v << w | tlo) = lds_idx(thi | tlo) + v * VSTEP, so one
-      // address register serves a source line's R reads (immediate offsets).
-      static_assert(w >= 4, "padding split");
-      constexpr uint32_t VSTEP = (1u << w) + (1u << (w - 4));
-      const uint32_t thi = (tau >> w) << (w + RHO), tlo = tau & ((1u << w) - 1);
-      const uint64_t* const sbase = src + lds_idx(0, thi | tlo, 0);
-      // Sources in groups of at most eight (conv_group); the groups' sum T
-      // (K <= 16: T >> 64 < 2^32 < t) takes one Montgomery reduction.
-      uint64_t tl[R], th[R];  // T = tl + th 2^64
-      const uint32_t k1 = K < 8 ? K : 8;
-      conv_group<R, VSTEP, PITCH>(sbase, qhat_mont, qhat_mont30, nq, k, 0, k1, tl, th);
-      if (K > 8) {
-        uint64_t t2[R], u2[R];
-        conv_group<R, VSTEP, PITCH>(sbase, qhat_mont, qhat_mont30, nq, k, 8, K, t2, u2);
-#pragma unroll
-        for (int v = 0; v < R; ++v) {
-          tl[v] += t2[v];
-          th[v] += u2[v] + (tl[v] < t2[v]);
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < R; ++v) x[v] = redc_lazy(th[v], tl[v], q, qn);  // (0, 2q)
-    }
-#pragma unroll
-    for (int sp = 0; sp < NSP; ++sp) {
-      const int hi = S1 - RHO * sp;
-      const int w = hi >= RHO ? hi - RHO : 0;
-      const int bhi = hi - 1;
-      const uint32_t thi = (tau >> w) << (w + RHO), tlo = tau & ((1u << w) - 1);
-      if (sp > 0) {
+    uint64_t x[R], twx[2][R - 1], twy[2][R - 1];
+    fetch_twiddles<S1, RHO, false, 0, LPW == 1>(tw, 1, tau, twx[0], twy[0]);
+    __syncthreads();
+    if (k < nq) {
+      static_for<NSP>([&](auto spc) {
+        constexpr int sp = decltype(spc)::value;
+        using W = SubPass<S1, RHO, false, sp>;
+        constexpr int w = W::w;
+        const uint32_t thi = (tau >> w) << (w + RHO), tlo = tau & ((1u << w) - 1);
+        if constexpr (sp + 1 < NSP)
+          fetch_twiddles<S1, RHO, false, sp + 1, LPW == 1>(tw, 1, tau, twx[(sp + 1) & 1],
+                                                           twy[(sp + 1) & 1]);
 #pragma unroll
         for (int v = 0; v < R; ++v) x[v] = line[lds_idx(0, thi | ((uint32_t)v << w) | tlo, 0)];
-      }
 #pragma unroll
-      for (int beta = bhi; beta >= w; --beta) {
-        const int d = 1 << (beta - w);
+        for (int k = RHO - 1; k >= 0; --k) {
+          const int beta = w + k, d = 1 << k;
+          if (beta > W::bhi) continue;
 #pragma unroll
-        for (int v = 0; v < R; ++v) {
-          if (v & d) continue;
-          const uint32_t u = thi | ((uint32_t)v << w) | tlo;
-          const uint32_t ti = (1u << (S1 - 1 - beta)) | (u >> (beta + 1));
-          const uint64_t wv = tw[2 * ti], ws = tw[2 * ti + 1];
-          fwd_butterfly(x[v], x[v + d], wv, ws, lm, fwd_reduces(16, 2, S1, beta));
+          for (int v = 0; v < R; ++v) {
+            if (v & d) continue;
+            const int ti = twiddle_at<RHO>(k, v);
+            fwd_butterfly(x[v], x[v + d], twx[sp & 1][ti], twy[sp & 1][ti], lm,
+                          fwd_reduces(16, 3, S1, beta));
+          }
         }
-      }
-      if (sp < NSP - 1) {
-        wave_lds_sync();
+        if (sp < NSP - 1) {
+          wave_lds_sync();
 #pragma unroll
-        for (int v = 0; v < R; ++v) line[lds_idx(0, thi | ((uint32_t)v << w) | tlo, 0)] = x[v];
-        wave_lds_sync();
-      } else {
-        // Last window (bits 0 .. RHO-1): rows R tau + v, one blocked run.
-        uint64_t* g = y + (size_t)kpos * N + blocked_off<S2>(R * tau, col);
+          for (int v = 0; v < R; ++v) line[lds_idx(0, thi | ((uint32_t)v << w) | tlo, 0)] = x[v];
+          wave_lds_sync();
+        } else {
+          // Last window (bits 0 .. RHO-1): rows R tau + v, one blocked run.
+          uint64_t* g = y + (size_t)kpos * N + blocked_off<S2>(R * tau, col);
 #pragma unroll
-        for (int v = 0; v < R; ++v) g[v] = x[v];
-      }
+          for (int v = 0; v < R; ++v) g[v] = x[v];
+        }
+      });
     }
+    if (k0 + nl < nq) __syncthreads();  // the next batch overwrites the lines
   }
 }
 
-template <int S1, int S2, int NW>
-__global__ void __launch_bounds__(64 * NW)
+template <int S1, int S2>
+__global__ void __launch_bounds__(1024)
     k_convert_mid(const MidArgs a, const ModConst* __restrict__ mc,
                   const uint64_t* __restrict__ tw_inv, const uint64_t* __restrict__ tw_fwd) {
-  extern __shared__ uint64_t lds_dyn[];
+  extern __shared__ __align__(16) uint64_t lds_dyn[];
   // Tiles in XCD order: workgroup i runs on XCD i % 8, and each XCD takes a
   // contiguous range of (poly, column) tiles, so neighbouring columns, which
   // share cache lines of the blocked layout, meet in one L2.
   const uint32_t per = gridDim.x / 8;
   const uint32_t tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
-  convert_mid_body<S1, S2, NW>(a, mc, tw_inv, tw_fwd, tile, lds_dyn);
+  convert_mid_body<S1, S2>(a, mc, tw_inv, tw_fwd, tile, blockDim.x / 64, lds_dyn);
 }
 
-template <int S1, int NW>
-size_t mid_lds_bytes(uint32_t K) {
-  return (size_t)(K + mid_lines<S1, NW>()) * mid_pitch<S1>() * 8;
+// LDS of a workgroup of nw waves: target constants (groups of four targets),
+// source lines, lines in flight.
+template <int S1>
+size_t mid_lds_bytes(uint32_t nsrc, uint32_t ndst, uint32_t nw) {
+  const size_t nl = (size_t)nw * (64 / mid_lanes_per_line<S1>());
+  return (size_t)((ndst + 3) / 4) * 4 * sizeof(MidTarget) + (nsrc + nl) * mid_pitch<S1>() * 8;
 }
 
-// Launches with fewer (poly, column) tiles than this use 8-wave workgroups.
-constexpr uint32_t MID_SMALL_TILES = 4096;
-// Launches of at most this many tiles (one ciphertext's ModUp or ModDown)
-// use 16-wave workgroups.
-constexpr uint32_t MID_TINY_TILES = 1024;
+// Waves per workgroup: 8, so that the source lines of a tile are done in one
+// or two rounds and three workgroups fit a CU (N = 2^16, us a call against 4 /
+// 16 waves: 30 ModDowns at 24 limbs 1553 / 1587 / 1693 for the whole step,
+// one product at 37 limbs 311 / 341 / 324); 16 at N = 2^17, whose lines of 512
+// rows leave one workgroup a CU either way (765 / 817 with 8).
+template <int S1>
+constexpr uint32_t mid_waves() {
+  return S1 == 9 ? 16 : 8;
+}
 
 template <int S1, int S2>
 void launch_mid(Context& c, const char* name, const MidArgs& a, uint32_t npoly,
-                uint32_t max_src) {
+                uint32_t max_src, uint32_t max_dst) {
   const uint32_t tiles = npoly << S2;
-  if (tiles <= MID_TINY_TILES && mid_lds_bytes<S1, 16>(max_src) <= c.lds_per_block) {
-    FHE_LAUNCH(c, name, (k_convert_mid<S1, S2, 16>), dim3(tiles), dim3(1024),
-               (mid_lds_bytes<S1, 16>(max_src)), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
-    return;
-  }
-  if (tiles < MID_SMALL_TILES && mid_lds_bytes<S1, 8>(max_src) <= c.lds_per_block) {
-    FHE_LAUNCH(c, name, (k_convert_mid<S1, S2, 8>), dim3(tiles), dim3(512),
-               (mid_lds_bytes<S1, 8>(max_src)), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
-    return;
-  }
-  FHE_LAUNCH(c, name, (k_convert_mid<S1, S2, 4>), dim3(tiles), dim3(256),
-             (mid_lds_bytes<S1, 4>(max_src)), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
+  uint32_t nw = mid_waves<S1>();
+  while (nw > 4 && mid_lds_bytes<S1>(max_src, max_dst, nw) > c.lds_per_block) nw /= 2;
+  FHE_LAUNCH(c, name, (k_convert_mid<S1, S2>), dim3(tiles), dim3(64 * nw),
+             (mid_lds_bytes<S1>(max_src, max_dst, nw)), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
 }
 
 // The target order of `pl` must be the one MidPlan describes (checked).
@@ -340,15 +347,15 @@ MidPlan mid_plan(const Context& c, const ConvPlan& pl, uint32_t src_mod0, uint32
     if (pl.dst_idx[k] != (pos < qlimbs ? pos : c.L + (pos - qlimbs)))
       throw ArgError("conversion plan target order");
   }
-  return MidPlan{pl.d_src_scale, pl.d_qhat_mont, pl.d_qhat_mont30, pl.nsrc, pl.ndst,
-                 src_mod0, src_limb0, skip_at, skip_len, qlimbs};
+  return MidPlan{pl.d_src_scale, pl.d_bytes, pl.nsrc,  pl.ndst, src_mod0,
+                 src_limb0,      skip_at,    skip_len, qlimbs};
 }
 
-bool mid_lds_fits(const Context& c, uint32_t nsrc) {
+bool mid_lds_fits(const Context& c, uint32_t nsrc, uint32_t ndst) {
   switch (c.log_n) {
-    case 13: case 14: return mid_lds_bytes<7, 4>(nsrc) <= c.lds_per_block;
-    case 15: case 16: return mid_lds_bytes<8, 4>(nsrc) <= c.lds_per_block;
-    case 17: return mid_lds_bytes<9, 4>(nsrc) <= c.lds_per_block;
+    case 13: case 14: return mid_lds_bytes<7>(nsrc, ndst, 4) <= c.lds_per_block;
+    case 15: case 16: return mid_lds_bytes<8>(nsrc, ndst, 4) <= c.lds_per_block;
+    case 17: return mid_lds_bytes<9>(nsrc, ndst, 4) <= c.lds_per_block;
     default: return false;
   }
 }
@@ -367,7 +374,7 @@ bool below_2_60_all(const Context& c, uint32_t nq) {
 }  // namespace
 
 bool convert_mid_ok(const Context& c, uint32_t nq, uint32_t nsrc) {
-  return below_2_60_all(c, nq) && mid_lds_fits(c, nsrc);
+  return nsrc <= MAX_CONV_SRC && below_2_60_all(c, nq) && mid_lds_fits(c, nsrc, nq + c.K);
 }
 
 void moddown_mid(Context& c, const uint64_t* ext_p, uint64_t* y, uint32_t npoly, uint32_t nq,
@@ -382,7 +389,7 @@ void moddown_mid(Context& c, const uint64_t* ext_p, uint64_t* y, uint32_t npoly,
   a.L = c.L;
   switch (c.log_n) {
 #define CASE(LN, A, B) \
-  case LN: launch_mid<A, B>(c, "k_moddown_mid", a, npoly, c.K); return;
+  case LN: launch_mid<A, B>(c, "k_moddown_mid", a, npoly, c.K, nq); return;
     CASE(13, 7, 6) CASE(14, 7, 7) CASE(15, 8, 7) CASE(16, 8, 8) CASE(17, 9, 8)
 #undef CASE
     default: throw ArgError("unsupported ring dimension");
@@ -430,7 +437,7 @@ void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t
     FHE_LAUNCH(c, "ntt_inv_blocks_modup", (ntt_pass_modup_in<B>), dim3(tiles, count, nq),     \
                dim3(256), 0, coef.p, (size_t)nq * n, c.d_const, c.d_tw_inv, c.log_n, s1, sp,  \
                digits, c.alpha, nd, ne);                                                      \
-    launch_mid<A, B>(c, "k_modup_mid", a, count * nd, max_src);                               \
+    launch_mid<A, B>(c, "k_modup_mid", a, count * nd, max_src, nq + c.K);                     \
     FHE_LAUNCH(c, "ntt_fwd_blocks_modup", (ntt_pass_modup_out<B>),                            \
                dim3(tiles, count * nd, ne - w_last), dim3(256), 0, digits, (size_t)ne * n,    \
                c.d_const, c.d_tw_fwd, c.log_n, map, s1);                                      \
