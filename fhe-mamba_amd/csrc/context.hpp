@@ -47,6 +47,8 @@ struct ModConst {
   uint64_t r64_sh;     // Shoup companion of r64
   uint64_t ninv;       // N^-1 mod q
   uint64_t ninv_sh;
+  uint64_t wninv;      // N^-1 times the inverse transform's last twiddle
+  uint64_t wninv_sh;
   uint64_t r2;         // 2^128 mod q (to Montgomery form via redc)
   // 2^64 - q and 2^64 - 4q, read from memory so that the compiler keeps
   // additions of them (shoup_lazy4n, lazy_sub) instead of folding them back

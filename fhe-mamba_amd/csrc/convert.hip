@@ -14,7 +14,7 @@ __global__ void __launch_bounds__(256)
                       uint32_t log_n, uint32_t s_other, const SrcPtrs src, uint64_t* digits,
                       uint32_t alpha, uint32_t nd, uint32_t ne) {
   ntt_body<16, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, SrcLoad, LimbMap, false, true>(
-      coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, 0, PlainStore{},
+      coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, PlainStore{},
       SrcLoad{src.p, 1u << log_n, digits, alpha, nd, ne});
 }
 
@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256)
                        const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                        uint32_t log_n, DigitMap map, uint32_t s_other) {
   ntt_body<16, S, BLOCKS, false, RHO_EPILOGUE, PlainStore, PlainLoad, DigitMap, true, false>(
-      digits, poly_stride, mc, tw_all, log_n, map, s_other, 1, PlainStore{});
+      digits, poly_stride, mc, tw_all, log_n, map, s_other, PlainStore{});
 }
 
 // ---- Fused middle of ModUp and of a batched ModDown, N = 2^13 .. 2^17 ----
@@ -57,15 +57,6 @@ __global__ void __launch_bounds__(256)
 // after adding t_k.  Per output that is about 17 VALU instructions whatever
 // the number of sources, where 64-bit multiply-adds took 4 a source and 25.
 constexpr uint32_t MAX_CONV_SRC = 16;
-
-template <int S1>
-constexpr uint32_t mid_pitch() {
-  return (1u << S1) + (1u << S1) / 16 + 1;
-}
-template <int S1>
-constexpr int mid_lanes_per_line() {
-  return (1 << S1) / 4 < 64 ? (1 << S1) / 4 : 64;
-}
 
 // What one (poly, column) tile converts.  Poly p of the launch uses plan
 // p % nplan; its sources are limbs src_limb0 .. src_limb0 + nsrc - 1 of
@@ -209,45 +200,61 @@ __device__ __forceinline__ void convert_mid_body(const MidArgs& a, const ModCons
   const uint32_t ksteps = (K + 3) / 4, half = lane >> 5, col32 = lane & 31;
   const uint32_t ugrp = wave * UPW / BLKS, ublk = wave * UPW % BLKS;
   uint64_t* const line = work + (size_t)first * PITCH;
+  // 1 and 2^16 as values the compiler does not know: products with them are
+  // multiply-adds that sign- or zero-extend their 32-bit operand for free.
+  const int one = (int)mc[0].one, c16 = one << 16;
+  // The units of one group of four targets from KS four-source steps.
+  // Sources past K are lines of other data: they meet zero table bytes.
+  auto convert = [&](auto ksc, uint32_t tg) {
+    constexpr int KS = decltype(ksc)::value;
+    const v4i* const tab = reinterpret_cast<const v4i*>(pl.bytes) + (size_t)tg * KS * 64 + lane;
+    v4i ab[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) ab[ks] = tab[ks * 64];
+    MidTarget mt[2];
+#pragma unroll
+    for (int o = 0; o < 2; ++o) mt[o] = tgt[4 * tg + 2 * half + o];
+#pragma unroll
+    for (uint32_t u = 0; u < UPW; ++u) {
+      const uint32_t idx = lds_idx(0, 32 * (ublk + u) + col32, 0);
+      const uint64_t* const sp = src + 2 * half * PITCH + idx;
+      v16i acc = {};
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const v2u sv = {sp[4 * ks * PITCH], sp[(4 * ks + 1) * PITCH]};
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ab[ks], __builtin_bit_cast(v4i, sv), acc, 0,
+                                                    0, 0);
+      }
+      uint64_t* const dst = work + (4 * ugrp + 2 * half) * PITCH + idx;
+#pragma unroll
+      for (int o = 0; o < 2; ++o) {
+        const int p01 = acc[8 * o] + (acc[8 * o + 1] << 8);
+        const int p23 = acc[8 * o + 2] + (acc[8 * o + 3] << 8);
+        const int p45 = acc[8 * o + 4] + (acc[8 * o + 5] << 8);
+        const int p67 = acc[8 * o + 6] + (acc[8 * o + 7] << 8);
+        // T = lo + 2^32 (hi - q);  m t = -lo mod 2^32, and the carry of lo +
+        // m t out of its low word is that of m t + 2^32 - 1 (none for lo = 0)
+        const int64_t lo = (int64_t)p01 * one + (int64_t)p23 * c16;
+        int64_t hi = (int64_t)mt[o].q + (int64_t)p45 * one;
+        hi += (int64_t)p67 * c16;
+        const uint32_t q0 = (uint32_t)mt[o].q, q1 = (uint32_t)(mt[o].q >> 32);
+        const uint32_t m = (uint32_t)lo * mt[o].qinv_neg;
+        const uint64_t mq0 = (uint64_t)m * q0 + 0xffffffffull;
+        uint64_t r = (uint64_t)(hi + (int64_t)(int32_t)(lo >> 32) * one);
+        r += (mq0 >> 32) * (uint32_t)one;
+        r += (uint64_t)m * q1;
+        dst[o * PITCH] = r;
+      }
+    }
+  };
   for (uint32_t k0 = 0; k0 < nq; k0 += nl) {
     const uint32_t tg = k0 / 4 + ugrp;
     if (tg < groups) {
-      const v4i* const tab = reinterpret_cast<const v4i*>(pl.bytes) + (size_t)tg * ksteps * 64 + lane;
-      MidTarget mt[2];
-#pragma unroll
-      for (int o = 0; o < 2; ++o) mt[o] = tgt[4 * tg + 2 * half + o];
-#pragma unroll
-      for (uint32_t u = 0; u < UPW; ++u) {
-        const uint32_t row = 32 * (ublk + u) + col32;
-        const uint64_t* const sp = src + lds_idx(0, row, 0);
-        v16i acc = {};
-        for (uint32_t ks = 0; ks < ksteps; ++ks) {
-          const v4i ab = tab[ks * 64];
-          // sources past K meet zero table bytes; any line will do for them
-          const uint32_t i0 = 4 * ks + 2 * half, i1 = i0 + 1;
-          v2u sv;
-          sv.x = sp[(size_t)(i0 < K ? i0 : K - 1) * PITCH];
-          sv.y = sp[(size_t)(i1 < K ? i1 : K - 1) * PITCH];
-          acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(ab, __builtin_bit_cast(v4i, sv), acc, 0, 0,
-                                                      0);
-        }
-#pragma unroll
-        for (int o = 0; o < 2; ++o) {
-          const int p01 = acc[8 * o] + (acc[8 * o + 1] << 8);
-          const int p23 = acc[8 * o + 2] + (acc[8 * o + 3] << 8);
-          const int p45 = acc[8 * o + 4] + (acc[8 * o + 5] << 8);
-          const int p67 = acc[8 * o + 6] + (acc[8 * o + 7] << 8);
-          // T = L + 2^32 H;  r = (T + m q) / 2^32 + q
-          const int64_t L = (int64_t)p23 * 65536 + p01;
-          const int64_t H = (int64_t)p67 * 65536 + p45;
-          const uint32_t q0 = (uint32_t)mt[o].q, q1 = (uint32_t)(mt[o].q >> 32);
-          const uint32_t m = (uint32_t)L * mt[o].qinv_neg;
-          const uint64_t lo = (uint64_t)m * q0 + (uint32_t)L;  // low word 0
-          uint64_t r = mt[o].q + (uint64_t)H + (uint64_t)(L >> 32);
-          r += lo >> 32;
-          r += (uint64_t)m * q1;
-          work[(size_t)(4 * ugrp + 2 * half + o) * PITCH + lds_idx(0, row, 0)] = r;
-        }
+      switch (ksteps) {
+        case 1: convert(std::integral_constant<int, 1>{}, tg); break;
+        case 2: convert(std::integral_constant<int, 2>{}, tg); break;
+        case 3: convert(std::integral_constant<int, 3>{}, tg); break;
+        default: convert(std::integral_constant<int, 4>{}, tg); break;
       }
     }
     const uint32_t k = k0 + first;
@@ -298,8 +305,12 @@ __device__ __forceinline__ void convert_mid_body(const MidArgs& a, const ModCons
   }
 }
 
+// Register budget: seven waves per SIMD (72 VGPRs, no spill) at N2 = 256 keep
+// three workgroups on a CU: 1514 us for the 30-rotation step against 1530 at
+// six and 1593 at eight (spills).
 template <int S1, int S2>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(S1 == 9 ? 1024 : 512)
+    __attribute__((amdgpu_waves_per_eu(S1 == 9 ? 4 : S1 == 8 ? 7 : 6, 8)))
     k_convert_mid(const MidArgs a, const ModConst* __restrict__ mc,
                   const uint64_t* __restrict__ tw_inv, const uint64_t* __restrict__ tw_fwd) {
   extern __shared__ __align__(16) uint64_t lds_dyn[];

@@ -12,9 +12,9 @@ template <int LIM, int S, int ND, bool BLK>
 __global__ void __launch_bounds__(256)
     ntt_pass_ksk(uint64_t* __restrict__ data, size_t poly_stride, const ModConst* __restrict__ mc,
                  const uint64_t* __restrict__ tw_all, uint32_t log_n, uint32_t s_other,
-                 int last, const ModDownEpi epi) {
+                 const ModDownEpi epi) {
   ntt_body<LIM, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, KskLoad<ND, BLK>, LimbMap, false,
-           BLK>(data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), s_other, last,
+           BLK>(data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), s_other,
                 PlainStore{}, KskLoad<ND, BLK>{epi, 1u << log_n});
 }
 
@@ -26,7 +26,7 @@ __global__ void __launch_bounds__(256)
                      const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                      uint32_t log_n, uint32_t s_other, const ModDownEpi epi) {
   ntt_body<LIM, S, BLOCKS, false, RHO_EPILOGUE, EpiStore<ND, BLK>, PlainLoad, LimbMap, BLK>(
-      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, 1,
+      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other,
       EpiStore<ND, BLK>{epi, 1u << log_n, log_n});
 }
 
@@ -396,7 +396,7 @@ void launch_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq, uint32
 }
 
 template <int S, bool BLK = false>
-void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other, bool last,
+void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other,
                 const ModDownEpi& epi) {
   using G = Geo<S, RHO_EPILOGUE>;
   const uint32_t tiles = (1u << s_other) / (256 / G::TPL);
@@ -407,7 +407,7 @@ void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other, boo
     // Both polys of each key switch in one workgroup (blocked output, digits
     // 1..7, no final scaling): rows per workgroup = one blocked group.
     constexpr uint32_t pair_lines = 512u >> (S - 2);
-    if (!last && npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
+    if (npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
       const dim3 pgrid((1u << s_other) / pair_lines, npoly / 2, c.K);
       switch (epi.nd) {
 #define CASE(D)                                                                              \
@@ -426,7 +426,7 @@ void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other, boo
     auto go = [&](auto lim) {
       FHE_LAUNCH(c, name, (ntt_pass_ksk<decltype(lim)::value, S, decltype(nd)::value, BLK>),
                  grid, dim3(256), 0, ext, ps, c.d_const, c.d_tw_inv, c.log_n, s_other,
-                 (int)last, epi);
+                 epi);
     };
     if constexpr (BLK)
       go(std::integral_constant<int, 16>{});
@@ -462,7 +462,7 @@ void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uin
   switch (c.log_n) {
 #define CASE(LN, B)                                                \
   case LN:                                                         \
-    launch_ksk<B, true>(c, ext_p, npoly, s1, false, epi);  \
+    launch_ksk<B, true>(c, ext_p, npoly, s1, epi);         \
     moddown_mid(c, ext_p, y, npoly, nq, pl);                       \
     launch_moddown<B, true>(c, y, npoly, nq, s1, epi);     \
     return;
@@ -482,7 +482,7 @@ void ntt_inverse_ksk(Context& c, uint64_t* ext_p, uint32_t npoly, const ModDownE
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
   switch (s2) {
 #define CASE(S) \
-  case S: launch_ksk<S>(c, ext_p, npoly, s1, false, epi); break;
+  case S: launch_ksk<S>(c, ext_p, npoly, s1, epi); break;
     CASE(6) CASE(7) CASE(8)
 #undef CASE
     default: throw ArgError("unsupported block pass");

@@ -8,15 +8,14 @@ namespace {
 template <int LIM, int S, int KIND, bool INV, class Map>
 __global__ void __launch_bounds__(max_threads<KIND>())
     ntt_pass(uint64_t* __restrict__ data, size_t poly_stride, const ModConst* __restrict__ mc,
-             const uint64_t* __restrict__ tw_all, uint32_t log_n, Map map, uint32_t s_other,
-             int last) {
+             const uint64_t* __restrict__ tw_all, uint32_t log_n, Map map, uint32_t s_other) {
   ntt_body<LIM, S, KIND, INV, KIND == SINGLE ? RHO_SINGLE : RHO_PLAIN, PlainStore, PlainLoad, Map>(
-      data, poly_stride, mc, tw_all, log_n, map, s_other, last, PlainStore{});
+      data, poly_stride, mc, tw_all, log_n, map, s_other, PlainStore{});
 }
 
 template <int S, int KIND, bool INV, class Map>
 void launch_pass(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
-                 Map map, uint32_t s_other, bool last) {
+                 Map map, uint32_t s_other) {
   using G = Geo<S, KIND == SINGLE ? RHO_SINGLE : RHO_PLAIN>;
   const uint32_t lines = KIND == SINGLE ? 1 : 256 / G::TPL;
   const uint32_t threads = KIND == SINGLE ? G::TPL : 256;
@@ -30,7 +29,7 @@ void launch_pass(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
   with_lim(c, [&](auto lim) {
     FHE_LAUNCH(c, PASS_NAME, (ntt_pass<decltype(lim)::value, S, KIND, INV, Map>), grid,
                dim3(threads), 0, data, poly_stride, c.d_const, INV ? c.d_tw_inv : c.d_tw_fwd,
-               c.log_n, map, s_other, (int)last);
+               c.log_n, map, s_other);
   });
 }
 
@@ -38,7 +37,7 @@ template <bool INV, class Map = LimbMap>
 void launch_single(Context& c, uint64_t* data, uint32_t npoly, size_t ps, uint32_t nlimb, Map map) {
   switch (c.log_n) {
 #define CASE(S) \
-  case S: launch_pass<S, SINGLE, INV>(c, data, npoly, ps, nlimb, map, 0, true); break;
+  case S: launch_pass<S, SINGLE, INV>(c, data, npoly, ps, nlimb, map, 0); break;
     CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11) CASE(12)
 #undef CASE
     default: throw ArgError("unsupported ring dimension");
@@ -47,10 +46,10 @@ void launch_single(Context& c, uint64_t* data, uint32_t npoly, size_t ps, uint32
 
 template <bool INV, class Map = LimbMap>
 void launch_cols(Context& c, uint32_t s1, uint32_t s2, uint64_t* data, uint32_t npoly, size_t ps,
-                 uint32_t nlimb, Map map, bool last) {
+                 uint32_t nlimb, Map map) {
   switch (s1) {
 #define CASE(S) \
-  case S: launch_pass<S, COLS, INV>(c, data, npoly, ps, nlimb, map, s2, last); break;
+  case S: launch_pass<S, COLS, INV>(c, data, npoly, ps, nlimb, map, s2); break;
     CASE(7) CASE(8) CASE(9)
 #undef CASE
     default: throw ArgError("unsupported column pass");
@@ -59,10 +58,10 @@ void launch_cols(Context& c, uint32_t s1, uint32_t s2, uint64_t* data, uint32_t 
 
 template <bool INV, class Map = LimbMap>
 void launch_blocks(Context& c, uint32_t s1, uint32_t s2, uint64_t* data, uint32_t npoly, size_t ps,
-                   uint32_t nlimb, Map map, bool last) {
+                   uint32_t nlimb, Map map) {
   switch (s2) {
 #define CASE(S) \
-  case S: launch_pass<S, BLOCKS, INV>(c, data, npoly, ps, nlimb, map, s1, last); break;
+  case S: launch_pass<S, BLOCKS, INV>(c, data, npoly, ps, nlimb, map, s1); break;
     CASE(6) CASE(7) CASE(8)
 #undef CASE
     default: throw ArgError("unsupported block pass");
@@ -88,17 +87,17 @@ void ntt_forward_digits(Context& c, uint64_t* digits, uint32_t count, uint32_t n
     return;
   }
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
-  launch_cols<false>(c, s1, s2, digits, npoly, ps, slots, map, false);
-  launch_blocks<false>(c, s1, s2, digits, npoly, ps, slots, map, true);
+  launch_cols<false>(c, s1, s2, digits, npoly, ps, slots, map);
+  launch_blocks<false>(c, s1, s2, digits, npoly, ps, slots, map);
 }
 
 void ntt_cols(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
               LimbMap map, bool inverse) {
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
   if (inverse)
-    launch_cols<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map, true);
+    launch_cols<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
   else
-    launch_cols<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map, false);
+    launch_cols<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
 }
 
 void ntt_forward(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
@@ -110,8 +109,8 @@ void ntt_forward(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
     return;
   }
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
-  launch_cols<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map, false);
-  launch_blocks<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map, true);
+  launch_cols<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
+  launch_blocks<false>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
 }
 
 void ntt_forward_table(Context& c, uint64_t* const* table, uint32_t npoly, uint32_t nlimb) {
@@ -123,8 +122,8 @@ void ntt_forward_table(Context& c, uint64_t* const* table, uint32_t npoly, uint3
     return;
   }
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
-  launch_cols<false>(c, s1, s2, nullptr, npoly, 0, nlimb, map, false);
-  launch_blocks<false>(c, s1, s2, nullptr, npoly, 0, nlimb, map, true);
+  launch_cols<false>(c, s1, s2, nullptr, npoly, 0, nlimb, map);
+  launch_blocks<false>(c, s1, s2, nullptr, npoly, 0, nlimb, map);
 }
 
 void ntt_inverse(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
@@ -136,8 +135,8 @@ void ntt_inverse(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
     return;
   }
   const uint32_t s1 = (c.log_n + 1) / 2, s2 = c.log_n / 2;
-  launch_blocks<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map, false);
-  launch_cols<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map, true);
+  launch_blocks<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
+  launch_cols<true>(c, s1, s2, data, npoly, poly_stride, nlimb, map);
 }
 
 }  // namespace fhe

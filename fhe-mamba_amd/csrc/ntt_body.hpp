@@ -201,8 +201,7 @@ template <int LIM, int S, int KIND, bool INV, int RHO_, class Store, class Load 
 __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t poly_stride,
                                          const ModConst* __restrict__ mc,
                                          const uint64_t* __restrict__ tw_all, uint32_t log_n,
-                                         Map map, uint32_t s_other, int last,
-                                         const Store& store, const Load& load = Load{}) {
+                                         Map map, uint32_t s_other, const Store& store, const Load& load = Load{}) {
   using G = Geo<S, RHO_>;
   constexpr int RHO = G::RHO;
   constexpr int R = 1 << RHO;
@@ -220,6 +219,7 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
   // library's own calls) for the first pass of a transform, else what the
   // first pass leaves.
   constexpr bool FIRST = KIND == SINGLE || (KIND == COLS) != INV;
+  constexpr bool LAST = KIND == SINGLE || (KIND == COLS) == INV;
   constexpr int B0 = FIRST ? 4 : INV ? LIM / 2 : fwd_pass_bound(LIM);
   static_assert(INV || fwd_bound(LIM, B0, S, -1) <= fwd_pass_bound(LIM), "forward bound");
   const uint64_t* __restrict__ tw = tw_all + (size_t)midx * n * 2;
@@ -345,7 +345,7 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
     // contiguous (staged positions do not depend on the window), else with
     // the last one.
     constexpr bool kFinalContig = !INV && KIND != COLS;
-    if (Store::kPre && last && sp == (kFinalContig ? 0 : NSP - 1)) {
+    if (Store::kPre && LAST && sp == (kFinalContig ? 0 : NSP - 1)) {
       const size_t wg0 = ((size_t)blockIdx.x * LINES) << S;
       if constexpr (Store::kPair && PAIR && kFinalContig) {
 #pragma unroll
@@ -395,22 +395,28 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
         for (int v = 0; v < R; ++v) {
           if (v & d) continue;
           const int ti = twiddle_at<RHO>(k, v);
-          inv_butterfly(x[v], x[v + d], twx[sp & 1][ti], twy[sp & 1][ti], lm, LIM, bnd[v],
+          const bool scaled = LAST && beta == S - 1;
+          inv_butterfly(x[v], x[v + d], scaled ? mc[midx].wninv : twx[sp & 1][ti],
+                        scaled ? mc[midx].wninv_sh : twy[sp & 1][ti], lm, LIM, bnd[v],
                         bnd[v + d]);
         }
       }
     }
 
     if (sp == NSP - 1) {
-      if (last) {
-        if (!INV) {
+      if constexpr (LAST && !INV) {
 #pragma unroll
-          for (int v = 0; v < R; ++v)
-            x[v] = LIM == 16 ? reduce_est(x[v], lm.neg_q, mc[midx].rq) : reduce_8q(x[v], q);
-        } else {
-          const uint64_t ni = mc[midx].ninv, nis = mc[midx].ninv_sh;
+        for (int v = 0; v < R; ++v)
+          x[v] = LIM == 16 ? reduce_est(x[v], lm.neg_q, mc[midx].rq) : reduce_8q(x[v], q);
+      }
+      if constexpr (LAST && INV) {
+        // N^-1: the last stage's products carry it in their twiddle, so only
+        // its sums (the lower half of the window) are still to be scaled.
+        const uint64_t ni = mc[midx].ninv, nis = mc[midx].ninv_sh;
 #pragma unroll
-          for (int v = 0; v < R; ++v) x[v] = reduce_4q(shoup_lazy4(x[v], ni, nis, q), q);
+        for (int v = 0; v < R; ++v) {
+          if (v < R / 2) x[v] = shoup_acc(0, x[v], ni, nis, lm.neg_q, lm.one);
+          x[v] = lazy_sub(lazy_sub(x[v], lm.neg_q + lm.neg_q), lm.neg_q);
         }
       }
       if (contiguous || BLK_OUT) {
@@ -500,6 +506,17 @@ template <int S2>
 __device__ __forceinline__ size_t blocked_off(uint32_t b, uint32_t u) {
   constexpr uint32_t BLO = blocked_rows<S2>();
   return (size_t)(b / BLO) * ((size_t)BLO << S2) + (size_t)u * BLO + (b % BLO);
+}
+
+// LDS words between, and lanes of a wavefront on, the column lines of M = 2^S1
+// rows in kernels that keep whole columns in LDS.
+template <int S1>
+constexpr uint32_t mid_pitch() {
+  return (1u << S1) + (1u << S1) / 16 + 1;
+}
+template <int S1>
+constexpr int mid_lanes_per_line() {
+  return (1 << S1) / 4 < 64 ? (1 << S1) / 4 : 64;
 }
 
 // ModUp input: limb blockIdx.z of ciphertext blockIdx.y's c1, read from the

@@ -18,7 +18,7 @@ __global__ void __launch_bounds__(256)
                         const uint64_t* __restrict__ tw_all, uint32_t log_n, uint32_t s_other,
                         const RescalePtrs ptrs, uint32_t npoly, size_t poly_words, uint32_t l) {
   ntt_body<LIM, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, LastLimbLoad>(
-      last, (size_t)1 << log_n, mc, tw_all, log_n, LimbMap::contiguous(l), s_other, 0,
+      last, (size_t)1 << log_n, mc, tw_all, log_n, LimbMap::contiguous(l), s_other,
       PlainStore{}, LastLimbLoad{ptrs.a, npoly, poly_words, (size_t)l << log_n});
 }
 
@@ -28,7 +28,7 @@ __global__ void __launch_bounds__(256)
                           const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                           uint32_t log_n, uint32_t s_other, const LiftLoad ld) {
   ntt_body<LIM, S, COLS, false, RHO_EPILOGUE, PlainStore, LiftLoad>(
-      t, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, 0, PlainStore{}, ld);
+      t, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, PlainStore{}, ld);
 }
 
 template <int LIM, int S>
@@ -39,7 +39,7 @@ __global__ void __launch_bounds__(256)
                          const uint64_t* __restrict__ rs, uint32_t l, uint32_t L,
                          uint32_t npoly) {
   ntt_body<LIM, S, BLOCKS, false, RHO_EPILOGUE, RescaleStore>(
-      t, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, 1,
+      t, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other,
       RescaleStore{ptrs.a, ptrs.out, rs, 1u << log_n, l, L, npoly});
 }
 
@@ -51,7 +51,7 @@ __global__ void __launch_bounds__(256)
                           const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                           uint32_t log_n, uint32_t s_other, uint32_t l) {
   ntt_body<LIM, S, COLS, true, RHO_EPILOGUE, PlainStore, PlainLoad, LimbMap>(
-      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(l), s_other, 1, PlainStore{});
+      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(l), s_other, PlainStore{});
 }
 
 }  // namespace

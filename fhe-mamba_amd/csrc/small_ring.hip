@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
                    uint32_t log_n, const SrcPtrs src, uint64_t* digits, uint32_t alpha,
                    uint32_t nd, uint32_t ne) {
   ntt_body<LIM, S, SINGLE, true, RHO_SINGLE, PlainStore, SrcLoad>(
-      coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, 1, PlainStore{},
+      coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, PlainStore{},
       SrcLoad{src.p, 1u << log_n, digits, alpha, nd, ne});
 }
 
@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
   uint32_t pos, mod;
   if (!map.resolve(blockIdx.y, blockIdx.z, pos, mod)) return;
   ntt_body<LIM, S, SINGLE, false, RHO_SINGLE, PlainStore, ConvLoad, DigitMap>(
-      digits, poly_stride, mc, tw_all, log_n, map, 0, 1, PlainStore{}, ConvLoad{conv, mod});
+      digits, poly_stride, mc, tw_all, log_n, map, 0, PlainStore{}, ConvLoad{conv, mod});
 }
 
 template <int LIM, int S, int ND>
@@ -89,7 +89,7 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
     small_ksk(uint64_t* __restrict__ data, size_t poly_stride, const ModConst* __restrict__ mc,
               const uint64_t* __restrict__ tw_all, uint32_t log_n, const ModDownEpi epi) {
   ntt_body<LIM, S, SINGLE, true, RHO_SINGLE, PlainStore, KskLoad<ND>>(
-      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), 0, 1, PlainStore{},
+      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), 0, PlainStore{},
       KskLoad<ND>{epi, 1u << log_n});
 }
 
@@ -102,11 +102,11 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
   const EpiStore<ND> st{epi, 1u << log_n, log_n};
   if constexpr (CONV)
     ntt_body<LIM, S, SINGLE, false, RHO_SINGLE, EpiStore<ND>, ConvLoad>(
-        y, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, 1, st,
+        y, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, st,
         ConvLoad{conv, blockIdx.z});
   else
     ntt_body<LIM, S, SINGLE, false, RHO_SINGLE, EpiStore<ND>>(
-        y, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, 1, st);
+        y, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, st);
 }
 
 // Rescale: the last limb to coefficient form, then every other limb's centred
@@ -117,7 +117,7 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
                      const uint64_t* __restrict__ tw_all, uint32_t log_n, const RescalePtrs ptrs,
                      uint32_t npoly, size_t poly_words, uint32_t l) {
   ntt_body<LIM, S, SINGLE, true, RHO_SINGLE, PlainStore, LastLimbLoad>(
-      last, (size_t)1 << log_n, mc, tw_all, log_n, LimbMap::contiguous(l), 0, 1, PlainStore{},
+      last, (size_t)1 << log_n, mc, tw_all, log_n, LimbMap::contiguous(l), 0, PlainStore{},
       LastLimbLoad{ptrs.a, npoly, poly_words, (size_t)l << log_n});
 }
 
@@ -127,7 +127,7 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
                       uint32_t log_n, const LiftLoad ld, const RescalePtrs ptrs,
                       const uint64_t* __restrict__ rs, uint32_t l, uint32_t L, uint32_t npoly) {
   ntt_body<LIM, S, SINGLE, false, RHO_SINGLE, RescaleStore, LiftLoad>(
-      nullptr, 0, mc, tw_all, log_n, LimbMap::contiguous(0), 0, 1,
+      nullptr, 0, mc, tw_all, log_n, LimbMap::contiguous(0), 0,
       RescaleStore{ptrs.a, ptrs.out, rs, 1u << log_n, l, L, npoly}, ld);
 }
 
