@@ -218,7 +218,8 @@ Context::Context(uint32_t log_n_, const uint64_t* q, uint32_t num_q, const uint6
       rs[o] = ql;
       rs[o + 1] = inv_;
       rs[o + 2] = host_shoup(inv_, qi);
-      rs[o + 3] = host_shoup(ql, qi);
+      // the least multiple of q_i not below q_l / 2
+      rs[o + 3] = qi * std::max<uint64_t>(1, ((mods[l] >> 1) + qi - 1) / qi);
     }
   d_rescale = upload(rs);
 

@@ -147,7 +147,8 @@ struct Context {
   ModConst* d_const = nullptr;       // [L+K]
   uint64_t* d_tw_fwd = nullptr;      // [L+K][N][2]
   uint64_t* d_tw_inv = nullptr;      // [L+K][N][2]
-  // rescale: rs[l][i] = (q_l mod q_i, (q_l)^-1 mod q_i, Shoup) for i < l
+  // rescale: rs[l][i] = (q_l mod q_i, (q_l)^-1 mod q_i, Shoup, the least
+  // multiple of q_i not below q_l / 2) for i < l
   uint64_t* d_rescale = nullptr;     // [L][L][4]
   // ModDown: P^-1 mod q_i (value, Shoup)
   uint64_t* d_pinv_q = nullptr;      // [L][2]

@@ -45,3 +45,26 @@ def test_key_switch_bit_exact(log_n, L, qbits, K, pbits, dnum):
         for c, o in zip(ct3, many):
             assert np.array_equal(o.numpy(), orc.rescale(c))
     ctx.close()
+
+
+# Q bit sizes, last limb dropped first: primes of one chain, a last prime many
+# times (reduced after its lift) and too many times (four launches) the others.
+RESCALES = [(13, (59, 59, 59)), (14, (60, 45, 59)), (15, (60, 34, 60)), (16, (45, 59)),
+            (17, (60, 59, 59)), (11, (60, 40, 59)), (13, (61, 59, 59))]
+
+
+@pytest.mark.parametrize("log_n,bits", RESCALES)
+def test_rescale_moduli(log_n, bits):
+    q = []
+    for b in bits:
+        q += O.ntt_friendly_primes(log_n, b, 1, skip=q)
+    ctx, orc = F.Context(log_n, q, [], 1, sampling="seeded"), O.Ctx(log_n, q, [], 1)
+    rng = np.random.default_rng(19)
+    pats = edge_patterns(q, ctx.n)
+    half = pats[0].copy()  # last limb coefficient q_l / 2 and its neighbours
+    last = q[-1]
+    coef = np.array([last // 2, last // 2 + 1, last - 1, 0] * (ctx.n // 4), dtype=np.uint64)
+    half[-1] = orc.ntt_fwd(coef, len(q) - 1)
+    for a in [residues(rng, q, (2,), ctx.n), pats[1:3], np.stack([half, pats[3]])]:
+        assert np.array_equal(ctx.rescale(ctx.upload(a)).numpy(), orc.rescale(a))
+    ctx.close()
