@@ -200,6 +200,7 @@ Context::Context(uint32_t log_n_, const uint64_t* q, uint32_t num_q, const uint6
       while ((double)f > want) f = std::nextafter(f, 0.0f);
       mc.rq = f;
       mc.one = 1;
+      mc.lift60 = qi * (((1ull << 60) + qi - 1) / qi);
     }
   }
   lazy16 = true;

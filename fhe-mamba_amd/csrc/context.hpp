@@ -57,6 +57,7 @@ struct ModConst {
   uint64_t qinv;       // q^-1 mod 2^64 (redc_lazy)
   uint64_t neg_q8;     // 2^64 - 8q (lazy_sub at 8q; 0 when 8q >= 2^64)
   float rq;            // 2^32 / q (1 - 2^-20), rounded down (reduce_est)
+  uint64_t lift60;     // the least multiple of q not below 2^60 (decode)
   uint32_t one;        // 1, as a value the compiler does not know (shoup_acc)
 };
 
@@ -356,9 +357,16 @@ void ntt_inverse(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
 // pass of a forward transform or the last, scaled one of an inverse.
 void ntt_cols(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride, uint32_t nlimb,
               LimbMap map, bool inverse);
-// Forward NTT of npoly one-poly [nlimb][N] operands held in separate
-// allocations; `table` is a device array of their npoly base pointers.
-void ntt_forward_table(Context& c, uint64_t* const* table, uint32_t npoly, uint32_t nlimb);
+// Forward NTT of signed 64-bit coefficients coef [npoly][N], reduced mod each
+// limb as the first pass loads them, into data [npoly][nlimb][N] (limb j mod
+// limb0 + j), or into one-poly operands held in separate allocations whose
+// base pointers are `table`, a device array of npoly (limb j mod q_j).
+void ntt_forward_signed(Context& c, const int64_t* coef, uint64_t* data, uint32_t npoly,
+                        size_t poly_stride, uint32_t nlimb, uint32_t limb0);
+void ntt_forward_signed_table(Context& c, const int64_t* coef, uint64_t* const* table,
+                              uint32_t npoly, uint32_t nlimb);
+// Inverse NTT of one poly [nlimb][N] at src into data.
+void ntt_inverse_from(Context& c, const uint64_t* src, uint64_t* data, uint32_t nlimb);
 // Forward NTT of y [npoly][nq][N] (limb j mod q_j) whose last pass stores
 // through the ModDown epilogue instead of writing y back.
 void ntt_forward_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq,

@@ -71,116 +71,114 @@ std::pair<double*, double*> fft_tables(Context& c, uint32_t slots) {
   return {di, df};
 }
 
-// One stage of the special inverse FFT: (a, b) -> (a + b, (a - b) * w).
-// Vector blockIdx.y of a batch of `slots`-value vectors.
-__global__ void k_fft_inv_stage(double2* v, const double* tw, uint32_t slots, uint32_t len) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= slots / 2) return;
-  v += (size_t)blockIdx.y * slots;
-  const uint32_t h = len / 2, j = t % h, i = (t / h) * len + j;
-  const double2 a = v[i], b = v[i + h];
-  const double wr = tw[2 * (h - 1 + j)], wi = tw[2 * (h - 1 + j) + 1];
+// One butterfly of the special inverse FFT: (a, b) -> (a + b, (a - b) w), and
+// of the forward one: (u, b) -> (u + b w, u - b w).
+__device__ __forceinline__ void fft_inv_butterfly(double2& a, double2& b, double2 w) {
   const double vr = a.x - b.x, vi = a.y - b.y;
-  v[i] = make_double2(a.x + b.x, a.y + b.y);
-  v[i + h] = make_double2(vr * wr - vi * wi, vi * wr + vr * wi);
+  a = make_double2(a.x + b.x, a.y + b.y);
+  b = make_double2(vr * w.x - vi * w.y, vi * w.x + vr * w.y);
+}
+__device__ __forceinline__ void fft_fwd_butterfly(double2& u, double2& b, double2 w) {
+  const double vr = b.x * w.x - b.y * w.y, vi = b.y * w.x + b.x * w.y;
+  b = make_double2(u.x - vr, u.y - vi);
+  u = make_double2(u.x + vr, u.y + vi);
 }
 
-// One stage of the forward special FFT: (u, b) -> (u + b w, u - b w).
-__global__ void k_fft_fwd_stage(double2* v, const double* tw, uint32_t slots, uint32_t len) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= slots / 2) return;
-  v += (size_t)blockIdx.y * slots;
-  const uint32_t h = len / 2, j = t % h, i = (t / h) * len + j;
-  const double2 u = v[i], b = v[i + h];
-  const double wr = tw[2 * (h - 1 + j)], wi = tw[2 * (h - 1 + j) + 1];
-  const double vr = b.x * wr - b.y * wi, vi = b.y * wr + b.x * wi;
-  v[i] = make_double2(u.x + vr, u.y + vi);
-  v[i + h] = make_double2(u.x - vr, u.y - vi);
-}
-
-// The stages with len <= FFT_BLOCK pair elements inside aligned blocks of
-// FFT_BLOCK values, so one workgroup runs all of them on its block in LDS:
-// the same butterflies and twiddles as the per-stage kernels above, in the
-// same order per element, hence the same roundings.
+// The transforms run in two kernels, each bound by the latency of its chain of
+// dependent stages: the stages with len <= FFT_BLOCK pair elements inside
+// aligned blocks of FFT_BLOCK values, one workgroup a block in LDS, one
+// butterfly a lane and stage with every stage's twiddle loaded up front; the
+// longer ones pair elements a multiple of slots / 2^T apart, 2^T values a lane
+// in registers (32768 slots, forward, us: 12.4 + 4 x 4.4 as a block kernel of
+// 256 lanes and a kernel a stage, 7.5 + 4.2 as this).  The butterflies and the order of each
+// element's are those of the radix-2 definition, hence the same roundings.
 constexpr uint32_t FFT_BLOCK = 2048;
 
-// Inverse stages len = top, top / 2, ..., 2 on blocks of `top` values.
-__global__ void __launch_bounds__(256)
-    k_fft_inv_block(double2* v, const double* tw, uint32_t top) {
-  __shared__ double2 x[FFT_BLOCK];
-  double2* g = v + (size_t)blockIdx.x * top;
-  for (uint32_t k = threadIdx.x; k < top; k += blockDim.x) x[k] = g[k];
-  __syncthreads();
-  for (uint32_t len = top; len >= 2; len >>= 1) {
-    const uint32_t h = len / 2;
-    for (uint32_t t = threadIdx.x; t < top / 2; t += blockDim.x) {
-      const uint32_t j = t % h, i = (t / h) * len + j;
-      const double2 a = x[i], b = x[i + h];
-      const double wr = tw[2 * (h - 1 + j)], wi = tw[2 * (h - 1 + j) + 1];
-      const double vr = a.x - b.x, vi = a.y - b.y;
-      x[i] = make_double2(a.x + b.x, a.y + b.y);
-      x[i + h] = make_double2(vr * wr - vi * wi, vi * wr + vr * wi);
-    }
-    __syncthreads();
-  }
-  for (uint32_t k = threadIdx.x; k < top; k += blockDim.x) g[k] = x[k];
+// Values of one-slot vectors.
+__global__ void k_real_to_complex(double2* v, const double* v_in, uint32_t count) {
+  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < count) v[k] = make_double2(v_in[k], 0.0);
 }
 
-// Forward stages len = 2, 4, ..., top on blocks of `top` values.
-__global__ void __launch_bounds__(256)
-    k_fft_fwd_block(double2* v, const double* tw, uint32_t top) {
-  __shared__ double2 x[FFT_BLOCK];
-  double2* g = v + (size_t)blockIdx.x * top;
-  for (uint32_t k = threadIdx.x; k < top; k += blockDim.x) x[k] = g[k];
+// Stages len = 2^LOG, ..., 2 (inverse) or 2, ..., 2^LOG (forward) on blocks of
+// 2^LOG values.  v_in: the inverse transform's input as real values.
+template <int LOG, bool INV>
+__global__ void __launch_bounds__(1024)
+    k_fft_block(double2* v, const double* v_in, const double* tw) {
+  constexpr uint32_t top = 1u << LOG;
+  __shared__ double2 x[top];
+  const uint32_t t = threadIdx.x;
+  const size_t g0 = (size_t)blockIdx.x * top;
+  const double2* const tw2 = reinterpret_cast<const double2*>(tw);
+  double2 w[LOG];
+#pragma unroll
+  for (int s = 0; s < LOG; ++s) w[s] = tw2[(1u << s) - 1 + (t & ((1u << s) - 1))];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t k = t + h * (top / 2);
+    x[k] = v_in ? make_double2(v_in[g0 + k], 0.0) : v[g0 + k];
+  }
   __syncthreads();
-  for (uint32_t len = 2; len <= top; len <<= 1) {
-    const uint32_t h = len / 2;
-    for (uint32_t t = threadIdx.x; t < top / 2; t += blockDim.x) {
-      const uint32_t j = t % h, i = (t / h) * len + j;
-      const double2 u = x[i], b = x[i + h];
-      const double wr = tw[2 * (h - 1 + j)], wi = tw[2 * (h - 1 + j) + 1];
-      const double vr = b.x * wr - b.y * wi, vi = b.y * wr + b.x * wi;
-      x[i] = make_double2(u.x + vr, u.y + vi);
-      x[i + h] = make_double2(u.x - vr, u.y - vi);
-    }
+#pragma unroll
+  for (int i = 0; i < LOG; ++i) {
+    const int s = INV ? LOG - 1 - i : i;  // h = len / 2 = 2^s
+    const uint32_t h = 1u << s, a = ((t >> s) << (s + 1)) | (t & (h - 1));
+    double2 p = x[a], q = x[a + h];
+    if (INV)
+      fft_inv_butterfly(p, q, w[s]);
+    else
+      fft_fwd_butterfly(p, q, w[s]);
+    x[a] = p;
+    x[a + h] = q;
     __syncthreads();
   }
-  for (uint32_t k = threadIdx.x; k < top; k += blockDim.x) g[k] = x[k];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) v[g0 + t + h * (top / 2)] = x[t + h * (top / 2)];
+}
+
+// The T longest stages (len = slots, ..., slots / 2^(T-1) for the inverse, the
+// other way round for the forward transform) of vector blockIdx.y.
+template <int T, bool INV>
+__global__ void __launch_bounds__(64)
+    k_fft_top(double2* v, const double* v_in, const double* tw, uint32_t slots) {
+  const uint32_t B = slots >> T, t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= B) return;
+  v += (size_t)blockIdx.y * slots;
+  const double2* const tw2 = reinterpret_cast<const double2*>(tw);
+  double2 x[1 << T];
+#pragma unroll
+  for (int k = 0; k < 1 << T; ++k)
+    x[k] = v_in ? make_double2(v_in[(size_t)blockIdx.y * slots + t + k * B], 0.0) : v[t + k * B];
+#pragma unroll
+  for (int i = 0; i < T; ++i) {
+    const int s = INV ? T - 1 - i : i;  // pairs k, k + 2^s: h = 2^s B
+#pragma unroll
+    for (int k = 0; k < 1 << T; ++k) {
+      if (k & (1 << s)) continue;
+      const double2 w = tw2[((1u << s) * B - 1) + t + (k & ((1 << s) - 1)) * B];
+      if (INV)
+        fft_inv_butterfly(x[k], x[k + (1 << s)], w);
+      else
+        fft_fwd_butterfly(x[k], x[k + (1 << s)], w);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 1 << T; ++k) v[t + k * B] = x[k];
 }
 
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits) {
   return bits ? __brev(x) >> (32 - bits) : 0;
 }
 
-__device__ __forceinline__ uint64_t lift_signed(int64_t x, uint64_t q) {
-  if (x >= 0) return (uint64_t)x % q;
-  const uint64_t r = ((uint64_t)(-x)) % q;
-  return r ? q - r : 0;
-}
-
-// x mod q for |x| < 2^63 by a Barrett step with mu64 = floor(2^64 / q): the
-// quotient estimate mulhi(|x|, mu64) is at most 1 below the true quotient,
-// so one conditional subtraction completes the reduction.
-__device__ __forceinline__ uint64_t lift_signed_mc(int64_t x, const ModConst& m) {
-  const uint64_t a = x >= 0 ? (uint64_t)x : (uint64_t)0 - (uint64_t)x;
-  uint64_t r = a - mulhi64(a, m.mu64) * m.q;
-  r = r >= m.q ? r - m.q : r;
-  return (x >= 0 || r == 0) ? r : m.q - r;
-}
-
-// Round slot i of the transformed vector (read through the bit reversal)
-// and scatter its real / imaginary coefficient into limbs blockIdx.z,
-// blockIdx.z + gridDim.z, ...  With a table, vector blockIdx.y of the
-// batch goes to table[blockIdx.y].
-__global__ void k_round_lift(const double2* v, uint64_t* out, uint64_t* const* table,
-                             const ModConst* mc, uint32_t slots, uint32_t bits, uint32_t gap,
-                             uint32_t n, uint32_t nlimb, double scale, int* status) {
+// Round slot i of the transformed vector (read through the bit reversal) to
+// its real / imaginary coefficient of vector blockIdx.y; the other
+// coefficients of the slot's two gap blocks are zero.
+__global__ void k_round(const double2* v, int64_t* coef, uint32_t slots, uint32_t bits,
+                        uint32_t gap, uint32_t n, double scale, int* status) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= slots) return;
-  if (table) {
-    v += (size_t)blockIdx.y * slots;
-    out = table[blockIdx.y];
-  }
+  v += (size_t)blockIdx.y * slots;
+  coef += (size_t)blockIdx.y * n;
   const double2 x = v[brev_bits(i, bits)];
   const double a = (x.x / (double)slots) * scale, b = (x.y / (double)slots) * scale;
   const double lim = 4611686018427387904.0;  // 2^62
@@ -188,70 +186,113 @@ __global__ void k_round_lift(const double2* v, uint64_t* out, uint64_t* const* t
     if (status) atomicOr(status, 1);
     return;
   }
-  const int64_t ra = llround(a), rb = llround(b);
-  for (uint32_t j = blockIdx.z; j < nlimb; j += gridDim.z) {
-    uint64_t* o = out + (size_t)j * n;
-    o[(size_t)i * gap] = lift_signed_mc(ra, mc[j]);
-    o[(size_t)(i + slots) * gap] = lift_signed_mc(rb, mc[j]);
-    // the other coefficients of this slot's two gap blocks are zero
-    for (uint32_t z = 1; z < gap; ++z) {
-      o[(size_t)i * gap + z] = 0;
-      o[(size_t)(i + slots) * gap + z] = 0;
-    }
+  coef[(size_t)i * gap] = llround(a);
+  coef[(size_t)(i + slots) * gap] = llround(b);
+  for (uint32_t z = 1; z < gap; ++z) {
+    coef[(size_t)i * gap + z] = 0;
+    coef[(size_t)(i + slots) * gap + z] = 0;
   }
 }
 
 // Balanced Garner reconstruction of coefficient positions i*gap, i < 2 slots,
 // then division by the scale; writes complex slot inputs of the forward FFT
-// at bit-reversed positions.
-template <int MAXL>
-__global__ void k_crt_decode(const uint64_t* coef, double2* v, const ModConst* mc,
-                             const uint64_t* garner, const uint64_t* mods, uint32_t n,
-                             uint32_t nlimb, uint32_t L, uint32_t slots, uint32_t bits,
-                             uint32_t gap, double scale) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 2 * slots) return;
-  const size_t pos = (size_t)t * gap;
-  int64_t a[MAXL];
-  double val = 0.0;
-  for (uint32_t i = 0; i < nlimb; ++i) {
-    const uint64_t q = mc[i].q;
-    uint64_t x = coef[(size_t)i * n + pos];
-    for (uint32_t j = 0; j < i; ++j) {
-      const uint64_t aj = lift_signed(a[j], q);
-      x = shoup(sub_mod(x, aj, q), garner[((size_t)i * L + j) * 2],
-                garner[((size_t)i * L + j) * 2 + 1], q);
+// at bit-reversed positions.  Digit a_j, once known, is taken out of every
+// later residue, x_i = (x_i - a_j) q_j^-1 mod q_i: one Shoup product of
+// x_i - a_j plus a multiple of q_i.  The steps j are a chain, the updates of
+// one step are not: a workgroup holds 64 coefficients' residues in LDS and its
+// CRT_WAVES wavefronts share each step's limbs, one barrier a step.  Bound by
+// the latency of that chain (32768 slots, 24 limbs: 186 us with one residue
+// after the other and hardware division, 63 with one wavefront a workgroup,
+// 37 as this).
+constexpr uint32_t CRT_WAVES = 4;
+__global__ void __launch_bounds__(64 * CRT_WAVES)
+    k_crt_decode(const uint64_t* coef, double2* v, const ModConst* mc, const uint64_t* garner,
+                 uint32_t n, uint32_t nlimb, uint32_t L, uint32_t slots, uint32_t bits,
+                 uint32_t gap, double scale) {
+  extern __shared__ uint64_t xs[];  // [nlimb][64]
+  const uint32_t t = blockIdx.x * 64 + (threadIdx.x & 63);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool valid = t < 2 * slots;
+  uint64_t* const x = xs + (threadIdx.x & 63);
+  for (uint32_t i = wave; i < nlimb; i += CRT_WAVES)
+    x[i * 64] = valid ? coef[(size_t)i * n + (size_t)t * gap] : 0;
+  for (uint32_t j = 0; j + 1 < nlimb; ++j) {
+    __syncthreads();
+    const uint64_t r = x[j * 64], qj = mc[j].q;
+    const uint64_t a = r > (qj >> 1) ? r - qj : r;  // balanced, as a signed word
+#pragma unroll 2
+    for (uint32_t i = j + 1 + ((wave - j - 1) & (CRT_WAVES - 1)); i < nlimb; i += CRT_WAVES) {
+      const uint64_t* g = garner + ((size_t)i * L + j) * 2;
+      x[i * 64] = shoup(x[i * 64] + mc[i].lift60 - a, g[0], g[1], mc[i].q);
     }
-    a[i] = x > (q >> 1) ? (int64_t)x - (int64_t)q : (int64_t)x;
   }
-  val = (double)a[nlimb - 1];
-  for (int i = (int)nlimb - 2; i >= 0; --i) val = val * (double)mods[i] + (double)a[i];
+  __syncthreads();
+  if (wave != 0 || !valid) return;
+  double val = 0.0;
+  for (int i = (int)nlimb - 1; i >= 0; --i) {
+    const uint64_t r = x[i * 64], q = mc[i].q;
+    const double d = (double)(int64_t)(r > (q >> 1) ? r - q : r);
+    val = i == (int)nlimb - 1 ? d : val * (double)q + d;
+  }
   val = val / scale;
   const uint32_t slot = t < slots ? t : t - slots;
   double* dst = reinterpret_cast<double*>(v + brev_bits(slot, bits));
   dst[t < slots ? 0 : 1] = val;
 }
 
-// The special FFT of nvec contiguous vectors of `slots` values each.  The
-// block kernels' blocks of `top` values never straddle two vectors (top
-// divides slots), so they run over the batch as one array.
-void run_stages(Context& c, double2* v, const double* tw, uint32_t slots, bool inverse,
-                uint32_t nvec = 1) {
-  if (slots < 2) return;
-  const uint32_t threads = slots / 2 < TPB ? slots / 2 : TPB;
-  const uint32_t blocks = (slots / 2 + threads - 1) / threads;
-  const uint32_t top = slots < FFT_BLOCK ? slots : FFT_BLOCK;
-  const uint32_t bthreads = top / 2 < TPB ? top / 2 : TPB;
-  const uint32_t nblk = nvec * (slots / top);
-  if (inverse) {
-    for (uint32_t len = slots; len > top; len >>= 1)
-      FHE_LAUNCH(c, "k_fft_inv_stage", k_fft_inv_stage, dim3(blocks, nvec), dim3(threads), 0, v, tw, slots, len);
-    FHE_LAUNCH(c, "k_fft_inv_block", k_fft_inv_block, dim3(nblk), dim3(bthreads), 0, v, tw, top);
-  } else {
-    FHE_LAUNCH(c, "k_fft_fwd_block", k_fft_fwd_block, dim3(nblk), dim3(bthreads), 0, v, tw, top);
-    for (uint32_t len = 2 * top; len <= slots; len <<= 1)
-      FHE_LAUNCH(c, "k_fft_fwd_stage", k_fft_fwd_stage, dim3(blocks, nvec), dim3(threads), 0, v, tw, slots, len);
+template <bool INV>
+void launch_fft_block(Context& c, double2* v, const double* v_in, const double* tw, uint32_t log,
+                      uint32_t nblk) {
+  const char* name = INV ? "k_fft_inv_block" : "k_fft_fwd_block";
+  if (log == 0) {
+    if (v_in)
+      FHE_LAUNCH(c, "k_real_to_complex", k_real_to_complex, dim3((nblk + 63) / 64), dim3(64), 0, v,
+                 v_in, nblk);
+    return;
   }
+  switch (log) {
+#define CASE(G)                                                                               \
+  case G:                                                                                     \
+    FHE_LAUNCH(c, name, (k_fft_block<G, INV>), dim3(nblk), dim3(1u << (G - 1)), 0, v, v_in, tw); \
+    return;
+    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8) CASE(9) CASE(10) CASE(11)
+#undef CASE
+    default: throw ArgError("unsupported slot count");
+  }
+}
+template <bool INV>
+void launch_fft_top(Context& c, double2* v, const double* v_in, const double* tw, uint32_t slots,
+                    uint32_t log, uint32_t nvec) {
+  const char* name = INV ? "k_fft_inv_top" : "k_fft_fwd_top";
+  switch (log) {
+#define CASE(T)                                                                              \
+  case T:                                                                                    \
+    FHE_LAUNCH(c, name, (k_fft_top<T, INV>), dim3((slots >> T) / 64, nvec), dim3(64), 0, v, \
+               v_in, tw, slots);                                                             \
+    return;
+    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5)
+#undef CASE
+    default: throw ArgError("unsupported slot count");
+  }
+}
+
+// The special FFT of nvec contiguous vectors of `slots` values each, in v; the
+// inverse one may take its input as real values v_in instead.  The block
+// kernel's blocks never straddle two vectors (their size divides slots), so
+// it runs over the batch as one array.
+// One slot is its own transform.
+void run_stages_inv(Context& c, double2* v, const double* v_in, const double* tw, uint32_t slots,
+                    uint32_t nvec) {
+  const uint32_t log = ilog2(slots), blk = slots < FFT_BLOCK ? log : ilog2(FFT_BLOCK);
+  const uint32_t top = log - blk;
+  if (top) launch_fft_top<true>(c, v, v_in, tw, slots, top, nvec);
+  launch_fft_block<true>(c, v, top ? nullptr : v_in, tw, blk, nvec * (slots >> blk));
+}
+void run_stages_fwd(Context& c, double2* v, const double* tw, uint32_t slots) {
+  if (slots < 2) return;
+  const uint32_t log = ilog2(slots), blk = slots < FFT_BLOCK ? log : ilog2(FFT_BLOCK);
+  launch_fft_block<false>(c, v, nullptr, tw, blk, slots >> blk);
+  if (log > blk) launch_fft_top<false>(c, v, nullptr, tw, slots, log - blk, 1);
 }
 
 void check_slots(const Context& c, uint32_t slots) {
@@ -261,50 +302,69 @@ void check_slots(const Context& c, uint32_t slots) {
 
 }  // namespace
 
+// Copies `count` values (real parts alone when im is null) into dst, zeros
+// up to `slots`, and whether some |z|^2 does not stay below lim2 (NaN and
+// infinities do not).
+static bool stage_values(double* dst, const double* re, const double* im, uint32_t count,
+                         uint32_t slots, double lim2) {
+  int over = 0;
+  if (im) {
+    for (uint32_t j = 0; j < count; ++j) {
+      const double a = re[j], b = im[j];
+      dst[2 * j] = a;
+      dst[2 * j + 1] = b;
+      over |= !(a * a + b * b < lim2);
+    }
+    std::memset(dst + 2 * (size_t)count, 0, 2 * (size_t)(slots - count) * sizeof(double));
+  } else {
+    for (uint32_t j = 0; j < count; ++j) {
+      const double a = re[j];
+      dst[j] = a;
+      over |= !(a * a < lim2);
+    }
+    std::memset(dst + count, 0, (size_t)(slots - count) * sizeof(double));
+  }
+  return over != 0;
+}
+
 bool encode(Context& c, const double* re, const double* im, uint32_t count, uint32_t slots,
             double scale, uint32_t nlimb, uint64_t* out) {
   check_slots(c, slots);
   if (count > slots) throw ArgError("more values than slots");
   if (nlimb == 0 || nlimb > c.L) throw ArgError("bad limb count");
   if (!(scale > 0) || !std::isfinite(scale)) throw ArgError("scale must be positive");
-  const size_t bytes = 2 * (size_t)slots * sizeof(double);
+  const uint32_t parts = im ? 2 : 1;
+  const size_t bytes = parts * (size_t)slots * sizeof(double);
   const auto tw = fft_tables(c, slots);
-  Scratch v(c, 2 * (size_t)slots), st(c, 1);
+  // real inputs are uploaded to where the rounded coefficients go afterwards
+  Scratch v(c, 2 * (size_t)slots), coef(c, c.n), st(c, 1);
   // Range bound: each inverse-FFT stage maps (a, b) to (a + b, (a - b) w)
   // with |w| = 1, so an output's modulus is at most the sum of the inputs'
   // and, after the division by slots, at most the largest input modulus.
   // Inputs whose bound times the scale stays below 2^62 (the margin 2^-20
-  // is far above the transform's rounding) cannot fail k_round_lift's range
+  // is far above the transform's rounding) cannot fail k_round's range
   // check, so nothing waits for the device; other inputs read the check's
   // status back, which waits for the stream.
-  // |z|^2 < (2^62 (1 - 2^-20) / scale)^2 for every value, with NaN and
-  // infinities failing the comparison.
   const double lim = 4611686018427387904.0 * (1.0 - 0x1p-20) / scale;
   const double lim2 = lim * lim;
   bool checked = !(lim2 < INFINITY);
+  double* const dst = reinterpret_cast<double*>(im ? v.p : coef.p);
   {
     std::lock_guard<std::mutex> g(c.staging_mu);
     Context::Staging& sg = c.staging_slot(bytes);
-    double* host = static_cast<double*>(sg.host);
-    int over = 0;
-    for (uint32_t j = 0; j < count; ++j) {
-      const double a = re[j], b = im ? im[j] : 0.0;
-      host[2 * j] = a;
-      host[2 * j + 1] = b;
-      over |= !(a * a + b * b < lim2);
-    }
-    checked = checked || over;
-    std::memset(host + 2 * (size_t)count, 0, bytes - 2 * (size_t)count * sizeof(double));
-    hip_check(hipMemcpyAsync(v.p, host, bytes, hipMemcpyHostToDevice, c.stream),
+    checked |= stage_values(static_cast<double*>(sg.host), re, im, count, slots, lim2);
+    hip_check(hipMemcpyAsync(dst, sg.host, bytes, hipMemcpyHostToDevice, c.stream),
               "encode upload");
     hip_check(hipEventRecord(sg.done, c.stream), "encode staging event");
   }
   if (checked) hip_check(hipMemsetAsync(st.p, 0, 8, c.stream), "encode status");
-  run_stages(c, reinterpret_cast<double2*>(v.p), tw.first, slots, true);
+  double2* const vv = reinterpret_cast<double2*>(v.p);
+  int64_t* const cf = reinterpret_cast<int64_t*>(coef.p);
+  run_stages_inv(c, vv, im ? nullptr : dst, tw.first, slots, 1);
   const uint32_t threads = slots < TPB ? slots : TPB;
-  // k_round_lift writes every coefficient of the nlimb limbs (the slots'
-  // positions and the zeros between them).
-  FHE_LAUNCH(c, "k_round_lift", k_round_lift, dim3((slots + threads - 1) / threads, 1, nlimb), dim3(threads), 0, reinterpret_cast<const double2*>(v.p), out, nullptr, c.d_const, slots, ilog2(slots), c.n / (2 * slots), c.n, nlimb, scale, checked ? reinterpret_cast<int*>(st.p) : nullptr);
+  FHE_LAUNCH(c, "k_round", k_round, dim3((slots + threads - 1) / threads), dim3(threads), 0, vv,
+             cf, slots, ilog2(slots), c.n / (2 * slots), c.n, scale,
+             checked ? reinterpret_cast<int*>(st.p) : nullptr);
   if (checked) {
     int status = 0;
     hip_check(hipMemcpyAsync(&status, st.p, sizeof(int), hipMemcpyDeviceToHost, c.stream),
@@ -312,7 +372,7 @@ bool encode(Context& c, const double* re, const double* im, uint32_t count, uint
     hip_check(hipStreamSynchronize(c.stream), "encode sync");
     if (status) return false;
   }
-  ntt_forward(c, out, 1, 0, nlimb, LimbMap::contiguous(0));
+  ntt_forward_signed(c, cf, out, 1, 0, nlimb, 0);
   return true;
 }
 
@@ -330,15 +390,28 @@ bool encode_many(Context& c, const double* re, const double* im, uint32_t count,
   constexpr uint32_t kChunk = 16;
   for (uint32_t r0 = 0; r0 < nvec; r0 += kChunk) {
     const uint32_t m = nvec - r0 < kChunk ? nvec - r0 : kChunk;
+    const size_t tab_words = (m + 1) & ~1u, vec_words = (im ? 2 : 1) * (size_t)slots;
+    const size_t words = tab_words + m * vec_words;
     bool over = !(lim2 < INFINITY);
-    for (uint32_t r = r0; r < r0 + m && !over; ++r)
-      for (uint32_t j = 0; j < count; ++j) {
-        const double a = re[(size_t)r * count + j], b = im ? im[(size_t)r * count + j] : 0.0;
-        if (!(a * a + b * b < lim2)) {
-          over = true;
-          break;
-        }
+    // real inputs are uploaded to where the rounded coefficients go afterwards
+    const size_t coef_words = m * (size_t)c.n, fft_words = m * 2 * (size_t)slots;
+    Scratch buf(c, tab_words + (im ? fft_words : coef_words)), other(c, im ? coef_words : fft_words);
+    uint64_t* const vals = buf.p + tab_words;
+    {
+      std::lock_guard<std::mutex> g(c.staging_mu);
+      Context::Staging& sg = c.staging_slot(words * 8);
+      uint64_t* host = static_cast<uint64_t*>(sg.host);
+      for (uint32_t r = 0; r < m; ++r) host[r] = reinterpret_cast<uint64_t>(outs[r0 + r]);
+      double* hv = reinterpret_cast<double*>(host + tab_words);
+      for (uint32_t r = 0; r < m && !over; ++r)
+        over = stage_values(hv + r * vec_words, re + (size_t)(r0 + r) * count,
+                            im ? im + (size_t)(r0 + r) * count : nullptr, count, slots, lim2);
+      if (!over) {
+        hip_check(hipMemcpyAsync(buf.p, host, words * 8, hipMemcpyHostToDevice, c.stream),
+                  "encode upload");
+        hip_check(hipEventRecord(sg.done, c.stream), "encode staging event");
       }
+    }
     if (over) {
       // Values that may not fit take the checked single path, which
       // reports the first vector that fails.
@@ -348,35 +421,14 @@ bool encode_many(Context& c, const double* re, const double* im, uint32_t count,
           return false;
       continue;
     }
-    const size_t tab_words = (m + 1) & ~1u, vec_words = 2 * (size_t)slots;
-    const size_t words = tab_words + m * vec_words;
-    Scratch buf(c, words);
-    double2* v = reinterpret_cast<double2*>(buf.p + tab_words);
-    {
-      std::lock_guard<std::mutex> g(c.staging_mu);
-      Context::Staging& sg = c.staging_slot(words * 8);
-      uint64_t* host = static_cast<uint64_t*>(sg.host);
-      for (uint32_t r = 0; r < m; ++r) host[r] = reinterpret_cast<uint64_t>(outs[r0 + r]);
-      double* hv = reinterpret_cast<double*>(host + tab_words);
-      for (uint32_t r = 0; r < m; ++r) {
-        const double* rr = re + (size_t)(r0 + r) * count;
-        const double* ri = im ? im + (size_t)(r0 + r) * count : nullptr;
-        double* h = hv + r * vec_words;
-        for (uint32_t j = 0; j < count; ++j) {
-          h[2 * j] = rr[j];
-          h[2 * j + 1] = ri ? ri[j] : 0.0;
-        }
-        std::memset(h + 2 * (size_t)count, 0, (vec_words - 2 * (size_t)count) * sizeof(double));
-      }
-      hip_check(hipMemcpyAsync(buf.p, host, words * 8, hipMemcpyHostToDevice, c.stream),
-                "encode upload");
-      hip_check(hipEventRecord(sg.done, c.stream), "encode staging event");
-    }
-    uint64_t* const* table = reinterpret_cast<uint64_t* const*>(buf.p);
-    run_stages(c, v, tw.first, slots, true, m);
+    double2* const v = reinterpret_cast<double2*>(im ? vals : other.p);
+    int64_t* const cf = reinterpret_cast<int64_t*>(im ? other.p : vals);
+    const double* const in = im ? nullptr : reinterpret_cast<const double*>(vals);
+    run_stages_inv(c, v, in, tw.first, slots, m);
     const uint32_t threads = slots < TPB ? slots : TPB;
-    FHE_LAUNCH(c, "k_round_lift", k_round_lift, dim3((slots + threads - 1) / threads, m, nlimb), dim3(threads), 0, v, nullptr, table, c.d_const, slots, ilog2(slots), c.n / (2 * slots), c.n, nlimb, scale, nullptr);
-    ntt_forward_table(c, table, m, nlimb);
+    FHE_LAUNCH(c, "k_round", k_round, dim3((slots + threads - 1) / threads, m), dim3(threads), 0,
+               v, cf, slots, ilog2(slots), c.n / (2 * slots), c.n, scale, nullptr);
+    ntt_forward_signed_table(c, cf, reinterpret_cast<uint64_t* const*>(buf.p), m, nlimb);
   }
   return true;
 }
@@ -386,23 +438,31 @@ void decode(Context& c, const uint64_t* pt, uint32_t nlimb, uint32_t slots, doub
   check_slots(c, slots);
   if (nlimb == 0 || nlimb > c.L) throw ArgError("bad limb count");
   const auto tw = fft_tables(c, slots);
-  Scratch coef(c, (size_t)nlimb * c.n), v(c, 2 * (size_t)slots), mods(c, c.L);
-  hip_check(hipMemcpyAsync(coef.p, pt, (size_t)nlimb * c.n * 8, hipMemcpyDeviceToDevice,
-                           c.stream),
-            "decode copy");
-  hip_check(hipMemcpyAsync(mods.p, c.mods.data(), c.L * 8, hipMemcpyHostToDevice, c.stream),
-            "decode moduli");
-  ntt_inverse(c, coef.p, 1, 0, nlimb, LimbMap::contiguous(0));
-  const uint32_t cnt = 2 * slots, threads = cnt < 64 ? cnt : 64;
-  FHE_LAUNCH(c, "k_crt_decode", (k_crt_decode<64>), dim3((cnt + threads - 1) / threads), dim3(threads), 0, coef.p, reinterpret_cast<double2*>(v.p), c.d_const, c.d_garner, mods.p, c.n, nlimb, c.L, slots, ilog2(slots), c.n / (2 * slots), scale);
-  run_stages(c, reinterpret_cast<double2*>(v.p), tw.second, slots, false);
-  std::vector<double> host(2 * (size_t)slots);
-  hip_check(hipMemcpyAsync(host.data(), v.p, host.size() * 8, hipMemcpyDeviceToHost, c.stream),
-            "decode download");
+  Scratch coef(c, (size_t)nlimb * c.n), v(c, 2 * (size_t)slots);
+  double2* const vv = reinterpret_cast<double2*>(v.p);
+  ntt_inverse_from(c, pt, coef.p, nlimb);
+  FHE_LAUNCH(c, "k_crt_decode", k_crt_decode, dim3((2 * slots + 63) / 64), dim3(64 * CRT_WAVES),
+             (size_t)nlimb * 64 * 8, coef.p, vv, c.d_const, c.d_garner, c.n, nlimb, c.L,
+             slots, ilog2(slots), c.n / (2 * slots), scale);
+  run_stages_fwd(c, vv, tw.second, slots);
+  // The transform is waited for before the staging buffer is taken, which is
+  // held for the length of the copy alone.
   hip_check(hipStreamSynchronize(c.stream), "decode sync");
-  for (uint32_t j = 0; j < slots; ++j) {
-    re[j] = host[2 * j];
-    if (im) im[j] = host[2 * j + 1];
+  const size_t bytes = 2 * (size_t)slots * sizeof(double);
+  std::lock_guard<std::mutex> g(c.staging_mu);
+  Context::Staging& sg = c.staging_slot(bytes);
+  hip_check(hipMemcpyAsync(sg.host, v.p, bytes, hipMemcpyDeviceToHost, c.stream),
+            "decode download");
+  hip_check(hipEventRecord(sg.done, c.stream), "decode staging event");
+  hip_check(hipStreamSynchronize(c.stream), "decode download");
+  const double* const host = static_cast<const double*>(sg.host);
+  if (im) {
+    for (uint32_t j = 0; j < slots; ++j) {
+      re[j] = host[2 * j];
+      im[j] = host[2 * j + 1];
+    }
+  } else {
+    for (uint32_t j = 0; j < slots; ++j) re[j] = host[2 * j];
   }
 }
 

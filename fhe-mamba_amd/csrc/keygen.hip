@@ -11,9 +11,12 @@
 //   Galois key k    s_old = s, s_new = s(X^{k^-1})
 //   relin key       s_old = s^2, s_new = s
 //   encryption      (pk_b v + e0 + m, pk_a v + e1), v ternary
-// Uniform residues are drawn on the GPU (counter-based stream, one word per
-// thread); small secrets and errors are drawn on the host and lifted.
-#include <vector>
+// Uniform residues and the small samples (v, e) are drawn on the GPU, each
+// lane a block of the counter-based stream, and lifted by the transforms'
+// first pass; the secret is the caller's, in host memory.  Drawn on the host
+// the three samples of an encryption were 450 us of its 527 (N=2^16, 24
+// limbs), most of them with the device idle.
+#include <cstring>
 
 #include "ops.hpp"
 #include "sampling.hpp"
@@ -25,20 +28,53 @@ constexpr int TPB = 256;
 
 inline uint32_t tpb_for(const Context& c) { return c.n < TPB ? c.n : TPB; }
 
-// Signed coefficients -> residues for limbs idx0 .. idx0 + nlimb.
-__global__ void k_lift_signed(const int64_t* coef, uint64_t* out, const ModConst* mc, uint32_t n,
-                              uint32_t idx0) {
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t q = mc[idx0 + blockIdx.y].q;
-  const int64_t x = coef[e];
-  uint64_t r;
-  if (x >= 0) {
-    r = (uint64_t)x % q;
+// Small samples drawn by one launch: stream p gives out[p][0..n), ternary or
+// centred binomial (the host definitions of both are in sampling.hpp).
+constexpr uint32_t MAX_DRAWS = 3;
+struct SmallDraws {
+  Stream s[MAX_DRAWS];
+  uint32_t ternary;  // bit p: stream p is ternary
+};
+
+// Words 8t .. 8t+7 of stream blockIdx.y: one ChaCha20 block a thread.
+__global__ void k_small_samples(int64_t* out, uint32_t n, SmallDraws d) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, p = blockIdx.y;
+  const Stream& s = d.s[p];
+  const bool ternary = (d.ternary >> p) & 1;
+  uint64_t w[8];
+  if (s.secure) {
+    stream_block(s, t, w);
   } else {
-    const uint64_t m = ((uint64_t)(-x)) % q;
-    r = m ? q - m : 0;
+    for (int i = 0; i < 8; ++i) w[i] = draw(s.sm_key, 8ull * t + i);
   }
-  out[(size_t)blockIdx.y * n + e] = r;
+  int64_t* o = out + (size_t)p * n + 8ull * t;
+  for (int i = 0; i < 8; ++i) o[i] = ternary ? ternary_from(w[i]) : cbd_from(w[i]);
+}
+
+void launch_small(Context& c, int64_t* out, const SmallDraws& d, uint32_t count) {
+  const uint32_t blocks = c.n / 8, tpb = blocks < 64 ? blocks : 64;
+  FHE_LAUNCH(c, "k_small_samples", k_small_samples, dim3(blocks / tpb, count), dim3(tpb), 0, out,
+             c.n, d);
+}
+
+// Centred binomial errors of stream (seed, tag, index) in evaluation form
+// over the first nlimb moduli.
+void errors_to_eval(Context& c, uint64_t seed, uint64_t tag, uint64_t index, uint32_t nlimb,
+                    uint64_t* out) {
+  Scratch coef(c, c.n);
+  int64_t* const cf = reinterpret_cast<int64_t*>(coef.p);
+  SmallDraws d{};
+  d.s[0] = make_stream(c.sampling, seed, tag, index);
+  launch_small(c, cf, d, 1);
+  ntt_forward_signed(c, cf, out, 1, 0, nlimb, 0);
+}
+
+// Calls that draw randomness or read the caller's host memory cannot be
+// replayed from a graph.
+void refuse_capture(Context& c, const char* what) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  hip_check(hipStreamIsCapturing(c.stream, &st), what);
+  if (st != hipStreamCaptureStatusNone) hip_check(hipErrorStreamCaptureUnsupported, what);
 }
 
 // out[j][e] = uniform mod q_{mod0+j} from words 2e, 2e+1 of stream
@@ -70,16 +106,16 @@ void launch_uniform(Context& c, uint64_t* out, uint32_t nlimb, uint64_t seed, ui
              c.n, base, seed, tag, index_base, mod0);
 }
 
-// b = e - a * s (+ f * s_old when f is given); all [nlimb][N], limb j uses
-// modulus mod0 + j; f is a per-limb factor array (0 outside the digit).
+// b = e - a * s (+ f * s_old on limbs [f_begin, f_end)); all [nlimb][N], f a
+// per-limb factor array.
 __global__ void k_key_combine(uint64_t* b, const uint64_t* a, const uint64_t* s,
                               const uint64_t* e, const uint64_t* s_old, const uint64_t* f,
-                              const ModConst* mc, uint32_t n, uint32_t mod0) {
+                              uint32_t f_begin, uint32_t f_end, const ModConst* mc, uint32_t n) {
   const uint32_t x = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
-  const ModConst m = mc[mod0 + j];
+  const ModConst m = mc[j];
   const size_t o = (size_t)j * n + x;
   uint64_t v = sub_mod(e[o], mul_mod(a[o], s[o], m), m.q);
-  if (f && f[j]) v = add_mod(v, mul_mod(f[j], s_old[o], m), m.q);
+  if (j >= f_begin && j < f_end) v = add_mod(v, mul_mod(f[j], s_old[o], m), m.q);
   b[o] = v;
 }
 
@@ -115,16 +151,6 @@ __global__ void k_square(uint64_t* out, const uint64_t* a, const ModConst* mc, u
   out[o] = mul_mod(a[o], a[o], mc[i]);
 }
 
-void signed_small_to_eval(Context& c, const std::vector<int64_t>& coef, uint32_t idx0,
-                          uint32_t nlimb, uint64_t* out) {
-  Scratch d(c, c.n);
-  hip_check(hipMemcpyAsync(d.p, coef.data(), c.n * 8, hipMemcpyHostToDevice, c.stream), "lift");
-  FHE_LAUNCH(c, "k_lift_signed", k_lift_signed, dim3(c.n / tpb_for(c), nlimb), dim3(tpb_for(c)), 0, reinterpret_cast<const int64_t*>(d.p), out, c.d_const, c.n, idx0);
-  ntt_forward(c, out, 1, 0, nlimb, LimbMap::contiguous(idx0));
-  // coef is host memory read by an async copy: finish before it can go away
-  hip_check(hipStreamSynchronize(c.stream), "lift sync");
-}
-
 }  // namespace
 
 void sample_secret_host(Context& c, uint64_t seed, int64_t* out) {
@@ -136,20 +162,30 @@ void sample_sparse_secret_host(Context& c, uint64_t seed, int64_t* out, uint32_t
 
 void signed_to_eval(Context& c, const int64_t* coef_host, uint32_t idx0, uint32_t nlimb,
                     uint64_t* out) {
-  std::vector<int64_t> v(coef_host, coef_host + c.n);
-  signed_small_to_eval(c, v, idx0, nlimb, out);
+  refuse_capture(c, "secret upload");
+  const size_t bytes = (size_t)c.n * 8;
+  Scratch coef(c, c.n);
+  {
+    // staged in pinned memory, so that nothing waits for the stream here and
+    // the caller's array is free when this returns
+    std::lock_guard<std::mutex> g(c.staging_mu);
+    Context::Staging& sg = c.staging_slot(bytes);
+    std::memcpy(sg.host, coef_host, bytes);
+    hip_check(hipMemcpyAsync(coef.p, sg.host, bytes, hipMemcpyHostToDevice, c.stream),
+              "secret upload");
+    hip_check(hipEventRecord(sg.done, c.stream), "secret staging event");
+  }
+  ntt_forward_signed(c, reinterpret_cast<const int64_t*>(coef.p), out, 1, 0, nlimb, idx0);
 }
 
 void keygen_public(Context& c, const int64_t* s_coef, uint64_t seed, uint64_t* pk) {
   const size_t n = c.n;
   Scratch s(c, c.L * n), e(c, c.L * n);
   signed_to_eval(c, s_coef, 0, c.L, s.p);
-  std::vector<int64_t> ec(n);
-  sample_cbd(make_stream(c.sampling, seed, TAG_PK_E, 0), ec.data(), c.n);
-  signed_small_to_eval(c, ec, 0, c.L, e.p);
+  errors_to_eval(c, seed, TAG_PK_E, 0, c.L, e.p);
   uint64_t* a = pk + (size_t)c.L * n;
   launch_uniform(c, a, c.L, seed, TAG_PK_A, 0, 0);
-  FHE_LAUNCH(c, "k_key_combine", k_key_combine, dim3(c.n / tpb_for(c), c.L), dim3(tpb_for(c)), 0, pk, a, s.p, e.p, nullptr, nullptr, c.d_const, c.n, 0u);
+  FHE_LAUNCH(c, "k_key_combine", k_key_combine, dim3(c.n / tpb_for(c), c.L), dim3(tpb_for(c)), 0, pk, a, s.p, e.p, nullptr, nullptr, 0u, 0u, c.d_const, c.n);
   hip_check(hipStreamSynchronize(c.stream), "keygen sync");
 }
 
@@ -157,27 +193,16 @@ void keygen_switch(Context& c, const uint64_t* s_old, const uint64_t* s_new, uin
                    uint64_t tag, uint64_t* key) {
   const size_t n = c.n;
   const uint32_t nm = c.L + c.K;
-  Scratch e(c, nm * n), f(c, nm);
-  std::vector<int64_t> ec(n);
-  std::vector<uint64_t> pmod(nm);
-  for (uint32_t i = 0; i < nm; ++i) {
-    uint64_t pm = 1 % c.mods[i];
-    for (uint32_t k = 0; k < c.K; ++k) pm = host_mulmod(pm, c.mods[c.L + k] % c.mods[i], c.mods[i]);
-    pmod[i] = pm;
-  }
-  std::vector<uint64_t> fac(nm);
+  Scratch e(c, nm * n);
   for (uint32_t j = 0; j < c.dnum; ++j) {
     const uint32_t s = j * c.alpha, end = s + c.alpha < c.L ? s + c.alpha : c.L;
-    sample_cbd(make_stream(c.sampling, seed, tag + TAG_KSK_E, j), ec.data(), c.n);
-    signed_small_to_eval(c, ec, 0, nm, e.p);
-    for (uint32_t i = 0; i < nm; ++i) fac[i] = (i >= s && i < end) ? pmod[i] : 0;
-    hip_check(hipMemcpyAsync(f.p, fac.data(), nm * 8, hipMemcpyHostToDevice, c.stream), "fac");
+    errors_to_eval(c, seed, tag + TAG_KSK_E, j, nm, e.p);
     uint64_t* b = key + ((size_t)j * 2) * nm * n;
     uint64_t* a = b + (size_t)nm * n;
     launch_uniform(c, a, nm, seed, tag + TAG_KSK_A, (uint64_t)j << 16, 0);
-    FHE_LAUNCH(c, "k_key_combine", k_key_combine, dim3(c.n / tpb_for(c), nm), dim3(tpb_for(c)), 0, b, a, s_new, e.p, s_old, f.p, c.d_const, c.n, 0u);
-    hip_check(hipStreamSynchronize(c.stream), "keygen sync");
+    FHE_LAUNCH(c, "k_key_combine", k_key_combine, dim3(c.n / tpb_for(c), nm), dim3(tpb_for(c)), 0, b, a, s_new, e.p, s_old, c.d_keyfac_out, s, end, c.d_const, c.n);
   }
+  hip_check(hipStreamSynchronize(c.stream), "keygen sync");
 }
 
 void keygen_galois(Context& c, const int64_t* s_coef, uint32_t galois, uint64_t seed,
@@ -199,16 +224,19 @@ void keygen_relin(Context& c, const int64_t* s_coef, uint64_t seed, uint64_t* ke
 
 void encrypt_pk(Context& c, const uint64_t* pk, const uint64_t* m, uint32_t nq, uint64_t seed,
                 uint64_t* ct) {
+  refuse_capture(c, "encrypt");
   const size_t n = c.n;
-  Scratch v(c, nq * n), e0(c, nq * n), e1(c, nq * n);
-  std::vector<int64_t> tmp(n);
-  sample_ternary(make_stream(c.sampling, seed, TAG_ENC_V, 0), tmp.data(), c.n);
-  signed_small_to_eval(c, tmp, 0, nq, v.p);
-  sample_cbd(make_stream(c.sampling, seed, TAG_ENC_E, 0), tmp.data(), c.n);
-  signed_small_to_eval(c, tmp, 0, nq, e0.p);
-  sample_cbd(make_stream(c.sampling, seed, TAG_ENC_E, 1), tmp.data(), c.n);
-  signed_small_to_eval(c, tmp, 0, nq, e1.p);
-  FHE_LAUNCH(c, "k_encrypt", k_encrypt, dim3(c.n / tpb_for(c), nq), dim3(tpb_for(c)), 0, ct, pk, v.p, e0.p, e1.p, m, c.d_const, c.n, nq, c.L);
+  Scratch coef(c, MAX_DRAWS * n), ve(c, MAX_DRAWS * nq * n);
+  int64_t* const cf = reinterpret_cast<int64_t*>(coef.p);
+  SmallDraws d{};
+  d.s[0] = make_stream(c.sampling, seed, TAG_ENC_V, 0);
+  d.s[1] = make_stream(c.sampling, seed, TAG_ENC_E, 0);
+  d.s[2] = make_stream(c.sampling, seed, TAG_ENC_E, 1);
+  d.ternary = 1;
+  launch_small(c, cf, d, 3);
+  ntt_forward_signed(c, cf, ve.p, 3, nq * n, nq, 0);
+  const uint64_t *v = ve.p, *e0 = v + nq * n, *e1 = e0 + nq * n;
+  FHE_LAUNCH(c, "k_encrypt", k_encrypt, dim3(c.n / tpb_for(c), nq), dim3(tpb_for(c)), 0, ct, pk, v, e0, e1, m, c.d_const, c.n, nq, c.L);
 }
 
 void decrypt(Context& c, const uint64_t* ct, uint32_t npoly, uint32_t nq, const int64_t* s_coef,

@@ -143,6 +143,18 @@ FHE_HD uint64_t uniform_from(uint64_t hi, uint64_t lo, uint64_t q) {
   return (uint64_t)(t >> 64);
 }
 
+// {0, 1, -1}[w mod 3]
+FHE_HD int64_t ternary_from(uint64_t w) {
+  const uint64_t d = w % 3;
+  return d == 0 ? 0 : (d == 1 ? 1 : -1);
+}
+
+// Centred binomial of eta = 21 from the low 42 bits.
+FHE_HD int64_t cbd_from(uint64_t w) {
+  return (int64_t)__builtin_popcountll(w & 0x1FFFFFull) -
+         (int64_t)__builtin_popcountll((w >> 21) & 0x1FFFFFull);
+}
+
 // Sequential reader of a stream on the host.
 class StreamReader {
  public:
@@ -165,10 +177,7 @@ class StreamReader {
 
 inline void sample_ternary(const Stream& st, int64_t* out, uint32_t n) {
   StreamReader r(st);
-  for (uint32_t i = 0; i < n; ++i) {
-    const uint64_t d = r.word(i) % 3;
-    out[i] = d == 0 ? 0 : (d == 1 ? 1 : -1);
-  }
+  for (uint32_t i = 0; i < n; ++i) out[i] = ternary_from(r.word(i));
 }
 
 // Exactly h nonzero coefficients, each +-1 (1 <= h <= n).
@@ -187,15 +196,6 @@ inline void sample_sparse_ternary(const Stream& st, int64_t* out, uint32_t n, ui
     out[idx[i]] = (r.word(2 * (uint64_t)i + 1) & 1) ? -1 : 1;
   }
   delete[] idx;
-}
-
-inline void sample_cbd(const Stream& st, int64_t* out, uint32_t n) {
-  StreamReader r(st);
-  for (uint32_t i = 0; i < n; ++i) {
-    const uint64_t d = r.word(i);
-    out[i] = (int64_t)__builtin_popcountll(d & 0x1FFFFFull) -
-             (int64_t)__builtin_popcountll((d >> 21) & 0x1FFFFFull);
-  }
 }
 
 }  // namespace fhe

@@ -356,10 +356,12 @@ class Context:
     def encode(self, values, slots: int, scale: float, nlimb: int, out=None) -> "Poly":
         v = np.asarray(values)
         re = np.ascontiguousarray(np.real(v), dtype=np.float64)
-        im = np.ascontiguousarray(np.imag(v), dtype=np.float64)
+        # real dtypes go without an imaginary part: half the upload
+        im = (None if v.dtype.kind in "fiub"
+              else np.ascontiguousarray(np.imag(v), dtype=np.float64))
         out = self._out(out, 1, nlimb)
-        call("fhe_encode", self.handle, _ptr(re), _ptr(im), len(v), slots, float(scale), nlimb,
-             out.handle)
+        call("fhe_encode", self.handle, _ptr(re), _ptr(im) if im is not None else None, len(v),
+             slots, float(scale), nlimb, out.handle)
         return out
 
     def encode_many(self, rows, slots: int, scale: float, nlimb: int) -> list:
@@ -377,10 +379,11 @@ class Context:
         return outs
 
     def decode(self, pt, slots: int, scale: float) -> np.ndarray:
-        re = np.zeros(slots)
-        im = np.zeros(slots)
+        re, im = np.empty(slots), np.empty(slots)
         call("fhe_decode", self.handle, pt.handle, slots, float(scale), _ptr(re), _ptr(im))
-        return re + 1j * im
+        out = np.empty(slots, dtype=np.complex128)
+        out.real, out.imag = re, im
+        return out
 
     # ---------------------------------------------------------- key material
     def keygen_secret(self, seed: int) -> np.ndarray:
