@@ -346,7 +346,12 @@ struct ModDownEpi {
   uint32_t ginv[MAX_KS_BATCH];
   size_t kl;                              // words per key component, (L+K) N
   uint32_t nd, ne, nq, L;
+  // raw: digits as modup_raw leaves them, own limbs read from own[r] [nq][N]
+  // (limb i belongs to digit i / alpha); nd <= RAW_MAX_DIGITS.
+  const uint64_t* own[MAX_KS_BATCH];
+  uint32_t raw, alpha;
 };
+constexpr uint32_t RAW_MAX_DIGITS = 4;
 
 // ---- kernel launchers (implemented in the .hip files) ----
 void ntt_forward(Context& c, uint64_t* data, uint32_t npoly, size_t poly_stride,
@@ -406,6 +411,10 @@ void rescale_fused_many(Context& c, uint64_t* const* outs, const uint64_t* const
 bool modup_fused_ok(const Context& c, uint32_t nq, uint32_t count);
 void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
                  uint64_t* digits);
+// ModUp without its last forward pass and without the digits' own limbs
+// (ModDownEpi::raw): converted limbs in the blocked layout.
+void modup_raw(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
+               uint64_t* digits);
 // Rings of at most 2^12 (small_ring.hip).  ModUp in two launches and ModDown's
 // conversion inside its last one, where the conversions have at most 8
 // sources; its first pass (`_ksk`) and last pass alone; rescale in two.

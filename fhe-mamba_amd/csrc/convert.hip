@@ -7,15 +7,15 @@ namespace {
 
 // First inverse pass of a fused ModUp: c1 of each ciphertext -> coef
 // (blocked layout).
-template <int S>
+template <int S, bool KEEP>
 __global__ void __launch_bounds__(256)
     ntt_pass_modup_in(uint64_t* __restrict__ coef, size_t poly_stride,
                       const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                       uint32_t log_n, uint32_t s_other, const SrcPtrs src, uint64_t* digits,
                       uint32_t alpha, uint32_t nd, uint32_t ne) {
-  ntt_body<16, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, SrcLoad, LimbMap, false, true>(
+  ntt_body<16, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, SrcLoad<KEEP>, LimbMap, false, true>(
       coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other, PlainStore{},
-      SrcLoad{src.p, 1u << log_n, digits, alpha, nd, ne});
+      SrcLoad<KEEP>{src.p, 1u << log_n, digits, alpha, nd, ne});
 }
 
 // Last forward pass of a fused ModUp over the digits' converted limbs
@@ -415,8 +415,8 @@ bool modup_fused_ok(const Context& c, uint32_t nq, uint32_t count) {
   return convert_mid_ok(c, nq, c.alpha);
 }
 
-void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
-                 uint64_t* digits) {
+static void modup_passes(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
+                         uint64_t* digits, bool raw) {
   if (!modup_fused_ok(c, nq, count)) throw ArgError("fused ModUp does not apply");
   const size_t n = c.n;
   const uint32_t ne = nq + c.K, nd = num_digits(c, nq);
@@ -445,19 +445,34 @@ void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t
   case LN: {                                                                                  \
     using G = Geo<B, RHO_EPILOGUE>;                                                           \
     const uint32_t tiles = (1u << s1) / (256 / G::TPL);                                       \
-    FHE_LAUNCH(c, "ntt_inv_blocks_modup", (ntt_pass_modup_in<B>), dim3(tiles, count, nq),     \
-               dim3(256), 0, coef.p, (size_t)nq * n, c.d_const, c.d_tw_inv, c.log_n, s1, sp,  \
-               digits, c.alpha, nd, ne);                                                      \
+    if (raw)                                                                                  \
+      FHE_LAUNCH(c, "ntt_inv_blocks_modup", (ntt_pass_modup_in<B, false>),                    \
+                 dim3(tiles, count, nq), dim3(256), 0, coef.p, (size_t)nq * n, c.d_const,     \
+                 c.d_tw_inv, c.log_n, s1, sp, nullptr, c.alpha, nd, ne);                      \
+    else                                                                                      \
+      FHE_LAUNCH(c, "ntt_inv_blocks_modup", (ntt_pass_modup_in<B, true>),                     \
+                 dim3(tiles, count, nq), dim3(256), 0, coef.p, (size_t)nq * n, c.d_const,     \
+                 c.d_tw_inv, c.log_n, s1, sp, digits, c.alpha, nd, ne);                       \
     launch_mid<A, B>(c, "k_modup_mid", a, count * nd, max_src, nq + c.K);                     \
-    FHE_LAUNCH(c, "ntt_fwd_blocks_modup", (ntt_pass_modup_out<B>),                            \
-               dim3(tiles, count * nd, ne - w_last), dim3(256), 0, digits, (size_t)ne * n,    \
-               c.d_const, c.d_tw_fwd, c.log_n, map, s1);                                      \
+    if (!raw)                                                                                 \
+      FHE_LAUNCH(c, "ntt_fwd_blocks_modup", (ntt_pass_modup_out<B>),                          \
+                 dim3(tiles, count * nd, ne - w_last), dim3(256), 0, digits, (size_t)ne * n,  \
+                 c.d_const, c.d_tw_fwd, c.log_n, map, s1);                                    \
     break;                                                                                    \
   }
     CASE(13, 7, 6) CASE(14, 7, 7) CASE(15, 8, 7) CASE(16, 8, 8) CASE(17, 9, 8)
 #undef CASE
     default: throw ArgError("unsupported ring dimension");
   }
+}
+
+void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
+                 uint64_t* digits) {
+  modup_passes(c, as, count, nq, digits, false);
+}
+void modup_raw(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
+               uint64_t* digits) {
+  modup_passes(c, as, count, nq, digits, true);
 }
 
 }  // namespace fhe

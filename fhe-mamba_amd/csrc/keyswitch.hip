@@ -364,8 +364,10 @@ void keyswitch_batch(Context& c, const uint64_t* digits, uint32_t nq,
   keyswitch_batch(c, dg, nq, keys, batch, outs);
 }
 
-void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
-                     const uint64_t* const* keys, uint32_t batch, const KeySwitchOut* outs) {
+// own: the switched polys, when the digits are modup_raw's (else null).
+static void switch_batch(Context& c, const uint64_t* const* digits, const uint64_t* const* own,
+                         uint32_t nq, const uint64_t* const* keys, uint32_t batch,
+                         const KeySwitchOut* outs) {
   if (batch == 0) return;
   if (batch > MAX_KS_BATCH) throw ArgError("key-switch batch too large");
   if (c.K == 0) throw ArgError("key switching needs special primes");
@@ -383,8 +385,11 @@ void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
   epi.ne = (uint32_t)ne;
   epi.nq = nq;
   epi.L = c.L;
+  epi.raw = own != nullptr;
+  epi.alpha = c.alpha;
   for (uint32_t r = 0; r < batch; ++r) {
     epi.digits[r] = digits[r];
+    epi.own[r] = own ? own[r] : nullptr;
     epi.key[r] = keys[r];
     epi.out[r] = outs[r].out;
     epi.add[r][0] = outs[r].add0;
@@ -407,6 +412,34 @@ void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
   ntt_forward_moddown(c, y.p, 2 * batch, nq, epi);
 }
 
+void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
+                     const uint64_t* const* keys, uint32_t batch, const KeySwitchOut* outs) {
+  switch_batch(c, digits, nullptr, nq, keys, batch, outs);
+}
+
+// One key switch each of count polys srcs[r]: their ModUp into dig
+// ([count][nd][nq+K][N]) and the batched ModDown.  Digits that one key switch
+// uses need no pass of their own over their last block stages: the two ModDown
+// passes that multiply them by the keys finish them in LDS, which saves
+// writing and re-reading them all (one rotation at N=2^16, us: 24 limbs, 3
+// digits 127 -> 114; N=2^17 multiplication of 41 limbs, 4 digits 735 -> 642).
+// Up to RAW_MAX_DIGITS digits, what two workgroups a CU have registers for.
+// Digits that several key switches share are finished once, by modup_batch.
+static void switch_each(Context& c, const uint64_t* const* srcs, uint32_t nq,
+                        const uint64_t* const* keys, uint32_t count, const KeySwitchOut* outs,
+                        uint64_t* dig) {
+  const uint32_t nd = num_digits(c, nq);
+  const size_t ct_words = (size_t)nd * (nq + c.K) * c.n;
+  std::vector<const uint64_t*> dg(count);
+  for (uint32_t r = 0; r < count; ++r) dg[r] = dig + r * ct_words;
+  const bool raw = nd <= RAW_MAX_DIGITS && modup_fused_ok(c, nq, count) && moddown_fused_ok(c, nq);
+  if (raw)
+    modup_raw(c, srcs, count, nq, dig);
+  else
+    modup_batch(c, srcs, count, nq, dig);
+  switch_batch(c, dg.data(), raw ? srcs : nullptr, nq, keys, count, outs);
+}
+
 void keyswitch_hoisted(Context& c, const uint64_t* digits, uint32_t nq,
                        const uint64_t* const* keys, const KeySwitchOut* outs, uint32_t count) {
   const size_t per_rot = 2 * (size_t)(c.K + nq) * c.n * 8;
@@ -419,8 +452,7 @@ void keyswitch_hoisted(Context& c, const uint64_t* digits, uint32_t nq,
 void keyswitch(Context& c, const uint64_t* a, uint32_t nq, const uint64_t* key,
                const KeySwitchOut& out) {
   Scratch dig(c, num_digits(c, nq) * (size_t)(nq + c.K) * c.n);
-  modup(c, a, nq, dig.p);
-  keyswitch_batch(c, dig.p, nq, &key, 1, &out);
+  switch_each(c, &a, nq, &key, 1, &out, dig.p);
 }
 
 void rotate(Context& c, uint64_t* out, const uint64_t* ct, uint32_t nq, const uint64_t* key,
@@ -442,10 +474,7 @@ static void keyswitch_many(Context& c, const uint64_t* const* srcs, uint32_t nq,
   for (uint32_t r0 = 0; r0 < count; r0 += batch) {
     const uint32_t b = std::min(batch, count - r0);
     Scratch dig(c, b * ct_words);
-    std::vector<const uint64_t*> dg(b);
-    for (uint32_t r = 0; r < b; ++r) dg[r] = dig.p + r * ct_words;
-    modup_batch(c, srcs + r0, b, nq, dig.p);
-    keyswitch_batch(c, dg.data(), nq, keys + r0, b, ko + r0);
+    switch_each(c, srcs + r0, nq, keys + r0, b, ko + r0, dig.p);
   }
 }
 
@@ -630,17 +659,14 @@ void linear_transform_many(Context& c, uint64_t* const* outs, const uint64_t* co
     inner(i, giants - 1, cur[i], false);
   }
   if (giants > 1) {
-    Scratch dig(c, (size_t)ncts * ct_words);
-    std::vector<const uint64_t*> c1(ncts), dg(ncts), keys(ncts, giant_keys[0]);
+    std::vector<const uint64_t*> c1(ncts), keys(ncts, giant_keys[0]);
     std::vector<KeySwitchOut> ko(ncts);
     for (int g = (int)giants - 2; g >= 0; --g) {
       for (uint32_t i = 0; i < ncts; ++i) {
         c1[i] = cur[i] + (size_t)nq * n;
-        dg[i] = dig.p + i * ct_words;
         ko[i] = KeySwitchOut{nxt[i], cur[i], nullptr, giant_galois[0]};
       }
-      modup_batch(c, c1.data(), ncts, nq, dig.p);
-      switch_all(dg, keys, ko);
+      keyswitch_many(c, c1.data(), nq, keys.data(), ko.data(), ncts);
       for (uint32_t i = 0; i < ncts; ++i) {
         inner(i, (uint32_t)g, nxt[i], true);
         std::swap(cur[i], nxt[i]);

@@ -48,6 +48,17 @@ __global__ void __launch_bounds__(256)
 // the kernel fits 64 VGPRs, four 8-wave workgroups per CU (0.84 -> 0.80 ms
 // for 30 key switches at N=2^16, 24 limbs, 3 digits, against forming them
 // first and keeping them in registers).
+//
+// RAW: a key switch's own digits (modup_raw), whose last forward pass runs here
+// too, two digits at a time through the same tile before y's; the finished
+// words stay in registers for the products.  Each round's loads are issued
+// ahead of the transform before them.  The digits' own pass over memory, and
+// the copy of their own limbs, are gone; this kernel and the P-limb one stay
+// bound by their reads, and by two 8-wave workgroups a CU (105-123 VGPRs;
+// three with spills were 12-20% slower over the whole key switch).  N=2^16, us:
+// relinearize + rescale of 37 limbs, 3 digits: the pass 41, ModDown's 52 + 24
+// before; 0, 68 + 33 now; 6 rotations of 21 limbs, 2 digits: 95, 119 + 68
+// before; 0, 150 + 107 now.
 // Rows per workgroup of the paired passes (one blocked group) and the LDS
 // words of their two-poly tile.
 template <int S>
@@ -59,50 +70,38 @@ constexpr uint32_t pair_lds_words() {
   return 2 * pair_lines<S>() * ((1u << S) + (1u << S) / 16 + 1);
 }
 
-// Body of the paired epilogue for the workgroup at row group bx of limb i of
-// key switch r, with its tile in lds (pair_lds_words<S>() words).
-template <int S, int ND>
-__device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y,
-                                                  const ModConst* __restrict__ mc,
-                                                  const uint64_t* __restrict__ tw_all,
-                                                  uint32_t log_n, uint32_t s_other,
-                                                  const ModDownEpi& e, uint32_t bx, uint32_t r,
-                                                  uint32_t i, uint64_t* lds_base) {
+// The forward block stages of H <= 2 blocked row groups src[h] (LINES rows)
+// of one modulus, with shared twiddles: the groups, fetched by fetch_group,
+// go to LDS, word p = u * LINES + row; the result, below 12q as from any pass,
+// is left there, each wavefront's rows written by it.  next() issues the loads
+// of what follows.  Every wavefront must be done with the tile before the call.
+__device__ __forceinline__ void fetch_group(ulonglong2 (&v)[2], const uint64_t* src) {
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    v[k] = *reinterpret_cast<const ulonglong2*>(src + (uint32_t)k * 1024u + 2 * threadIdx.x);
+}
+template <int S, int H, class Next>
+__device__ __forceinline__ void forward_groups(uint64_t* const (&lds)[2],
+                                               const ulonglong2 (&in)[2][2], const Next& next,
+                                               const uint64_t* __restrict__ tw, uint32_t twbase,
+                                               uint32_t tau, uint32_t line, const LazyMod& lm) {
   constexpr int RHO = 2, R = 4, TPL = 1 << (S - RHO), LINES = 512 / TPL;
   constexpr int NSP = (S + RHO - 1) / RHO;
   constexpr uint32_t LEN = 1u << S, PITCH = LEN + LEN / 16 + 1;
-  static_assert(TPL <= 64 && LINES * TPL == 512 && ND > 0 && ND <= 7, "pair epilogue");
-  uint64_t* const lds[2] = {lds_base, lds_base + LINES * PITCH};
-  const uint32_t n = 1u << log_n, tid = threadIdx.x;
-  const uint64_t q = mc[i].q;
-  const LazyMod lm = lazy_mod<16>(mc[i]);
-  const float rq = mc[i].rq;
-  const uint64_t* __restrict__ tw = tw_all + (size_t)i * n * 2;
-  const size_t ps = (size_t)e.nq * n, wg0 = ((size_t)bx * LINES) << S;
-  const uint32_t tau = tid % TPL, line = tid / TPL;
-  const uint32_t twbase = (1u << s_other) + bx * LINES + line;
-  // Key-product and store positions of this lane: two adjacent pairs in its
-  // wavefront's own 64R-word run (the wavefront's rows).
-  auto staged = [&](int k) -> uint32_t {
-    return (tid >> 6) * (64u * R) + (uint32_t)(k >> 1) * 128u + 2 * (tid & 63) + (k & 1);
-  };
-
-  // The blocked group of both polys into LDS, word p = u * LINES + row,
-  // two adjacent words per lane (16-byte loads).
+  const uint32_t tid = threadIdx.x;
 #pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint64_t* __restrict__ src = y + (size_t)(2 * r + h) * ps + (size_t)i * n + wg0;
+  for (int h = 0; h < H; ++h) {
 #pragma unroll
     for (int k = 0; k < R; k += 2) {
       const uint32_t p = (uint32_t)k * 512u + 2 * tid;
-      const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(src + p);
-      lds[h][lds_idx(p % LINES, p / LINES, PITCH)] = v.x;
-      lds[h][lds_idx((p + 1) % LINES, (p + 1) / LINES, PITCH)] = v.y;
+      lds[h][lds_idx(p % LINES, p / LINES, PITCH)] = in[h][k / 2].x;
+      lds[h][lds_idx((p + 1) % LINES, (p + 1) / LINES, PITCH)] = in[h][k / 2].y;
     }
   }
   __syncthreads();
+  next();
 
-  uint64_t x[2][R];
+  uint64_t x[H][R];
   uint64_t twx[2][R - 1], twy[2][R - 1];
   fetch_twiddles<S, RHO, false, 0, TPL == 64>(tw, twbase, tau, twx[0], twy[0]);
   static_for<NSP>([&](auto spc) {
@@ -114,8 +113,8 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
 #pragma unroll
     for (int v = 0; v < R; ++v) {
       const uint32_t u = thi | ((uint32_t)v << w) | tlo;
-      x[0][v] = lds[0][lds_idx(line, u, PITCH)];
-      x[1][v] = lds[1][lds_idx(line, u, PITCH)];
+#pragma unroll
+      for (int h = 0; h < H; ++h) x[h][v] = lds[h][lds_idx(line, u, PITCH)];
     }
     if constexpr (sp + 1 < NSP)
       fetch_twiddles<S, RHO, false, sp + 1, TPL == 64>(tw, twbase, tau, twx[(sp + 1) & 1],
@@ -130,7 +129,7 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
         const int ti = twiddle_at<RHO>(k, v);
         const uint64_t wv = twx[sp & 1][ti], ws = twy[sp & 1][ti];
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < H; ++h)
           fwd_butterfly(x[h][v], x[h][v + d], wv, ws, lm,
                         fwd_reduces(16, fwd_pass_bound(16), S, beta));
       }
@@ -139,11 +138,106 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
 #pragma unroll
     for (int v = 0; v < R; ++v) {
       const uint32_t u = thi | ((uint32_t)v << w) | tlo;
-      lds[0][lds_idx(line, u, PITCH)] = x[0][v];
-      lds[1][lds_idx(line, u, PITCH)] = x[1][v];
+#pragma unroll
+      for (int h = 0; h < H; ++h) lds[h][lds_idx(line, u, PITCH)] = x[h][v];
     }
   });
   wave_lds_sync();
+}
+
+// Position k of lane tid in the workgroup's rows, as the key products and
+// stores take them: two adjacent pairs in its wavefront's own run of rows.
+__device__ __forceinline__ uint32_t pair_staged(uint32_t tid, int k) {
+  return (tid >> 6) * 256u + (uint32_t)(k >> 1) * 128u + 2 * (tid & 63) + (k & 1);
+}
+
+// The last forward pass of M digits that ModUp left before it: dst[j] = words
+// at positions pair_staged of digit j's group (src(j), blocked), reduced.  Two
+// digits at a time through the tile, which the caller may overwrite on return.
+template <int S, int M, class Src, class Next>
+__device__ __forceinline__ void finish_digits(uint64_t* const (&lds)[2], ulonglong2 (&in)[2][2],
+                                              const Src& src, const Next& next,
+                                              const uint64_t* __restrict__ tw, uint32_t twbase,
+                                              uint32_t tau, uint32_t line, const LazyMod& lm,
+                                              float rq, ulonglong2 (&dst)[M][2]) {
+  constexpr uint32_t LEN = 1u << S, PITCH = LEN + LEN / 16 + 1;
+  static_for<(M + 1) / 2>([&](auto rd) {
+    constexpr int j0 = 2 * decltype(rd)::value, H = M - j0 < 2 ? 1 : 2;
+    if constexpr (j0 == 0) {
+#pragma unroll
+      for (int h = 0; h < H; ++h) fetch_group(in[h], src(h));
+    }
+    forward_groups<S, H>(
+        lds, in,
+        [&] {
+          if constexpr (j0 + 2 >= M) {
+            next();
+          } else {
+            constexpr int HN = M - j0 - 2 < 2 ? 1 : 2;
+#pragma unroll
+            for (int h = 0; h < HN; ++h) fetch_group(in[h], src(j0 + 2 + h));
+          }
+        },
+        tw, twbase, tau, line, lm);
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+#pragma unroll
+      for (int k = 0; k < 4; k += 2) {
+        const uint32_t p = pair_staged(threadIdx.x, k);
+        dst[j0 + h][k / 2] = ulonglong2{
+            reduce_est(lds[h][lds_idx(p >> S, p & (LEN - 1), PITCH)], lm.neg_q, rq),
+            reduce_est(lds[h][lds_idx((p + 1) >> S, (p + 1) & (LEN - 1), PITCH)], lm.neg_q, rq)};
+      }
+    }
+    __syncthreads();
+  });
+}
+
+// Body of the paired epilogue for the workgroup at row group bx of limb i of
+// key switch r, with its tile in lds (pair_lds_words<S>() words).
+template <int S, int ND, bool RAW>
+__device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y,
+                                                  const ModConst* __restrict__ mc,
+                                                  const uint64_t* __restrict__ tw_all,
+                                                  uint32_t log_n, uint32_t s_other,
+                                                  const ModDownEpi& e, uint32_t bx, uint32_t r,
+                                                  uint32_t i, uint64_t* lds_base) {
+  constexpr int RHO = 2, R = 4, TPL = 1 << (S - RHO), LINES = 512 / TPL;
+  constexpr uint32_t LEN = 1u << S, PITCH = LEN + LEN / 16 + 1;
+  static_assert(TPL <= 64 && LINES * TPL == 512 && ND > 0 && ND <= 7, "pair epilogue");
+  uint64_t* const lds[2] = {lds_base, lds_base + LINES * PITCH};
+  const uint32_t n = 1u << log_n, tid = threadIdx.x;
+  const uint64_t q = mc[i].q;
+  const LazyMod lm = lazy_mod<16>(mc[i]);
+  const float rq = mc[i].rq;
+  const uint64_t* __restrict__ tw = tw_all + (size_t)i * n * 2;
+  const size_t ps = (size_t)e.nq * n, wg0 = ((size_t)bx * LINES) << S;
+  const uint32_t tau = tid % TPL, line = tid / TPL;
+  const uint32_t twbase = (1u << s_other) + bx * LINES + line;
+  // RAW: digit j's words are formed here from ModUp's intermediate (its own
+  // limb, which needs no transform, comes from the source poly).  Slot j < M
+  // holds the converted digits in order, the last slot the limb's own digit.
+  constexpr int M = RAW ? ND - 1 : 0;
+  const size_t dstride = (size_t)e.ne * n;
+  const uint32_t own = RAW ? i / e.alpha : 0;
+  auto digit_of = [&](int slot) -> uint32_t {
+    return !RAW ? slot : slot == M ? own : (uint32_t)slot + ((uint32_t)slot >= own ? 1u : 0u);
+  };
+  ulonglong2 up[RAW && M > 0 ? M : 1][2];
+  ulonglong2 in[2][2];
+  auto fetch_y = [&] {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      fetch_group(in[h], y + (size_t)(2 * r + h) * ps + (size_t)i * n + wg0);
+  };
+  if constexpr (RAW && M > 0)
+    finish_digits<S, M>(
+        lds, in,
+        [&](int j) { return e.digits[r] + digit_of(j) * dstride + (size_t)i * n + wg0; },
+        fetch_y, tw, twbase, tau, line, lm, rq, up);
+  else
+    fetch_y();
+  forward_groups<S, 2>(lds, in, [] {}, tw, twbase, tau, line, lm);
 
   // Key products of both polys at this lane's positions, the digits' words
   // read once (16-byte loads, two positions each), plus the transform, out
@@ -151,21 +245,25 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
   const uint32_t gi = e.ginv[r];
   uint64_t* const out0 = e.out[r] + (size_t)i * n;
   uint64_t* const out1 = e.out[r] + ((size_t)e.nq + i) * n;
-  const size_t dstride = (size_t)e.ne * n, kstride = 2 * e.kl;
+  const size_t kstride = 2 * e.kl;
   const uint64_t* const a0 = e.add[r][0];
   const uint64_t* const a1 = e.add[r][1];
   const uint64_t qn = e.mc[i].qinv;
 #pragma unroll
   for (int k = 0; k < R; k += 2) {
-    const size_t s0 = wg0 + staged(k);
-    const uint64_t* dg = e.digits[r] + (size_t)i * n + s0;
+    const size_t s0 = wg0 + pair_staged(tid, k);
+    const uint64_t* dg = (RAW ? e.own[r] : e.digits[r]) + (size_t)i * n + s0;
     const uint64_t* kr = e.key[r] + (size_t)i * n + s0;
     ulonglong2 d[ND], k0[ND], k1[ND];
 #pragma unroll
     for (int j = 0; j < ND; ++j) {
-      d[j] = *reinterpret_cast<const ulonglong2*>(dg + j * dstride);
-      k0[j] = load_stream2(kr + j * kstride);
-      k1[j] = load_stream2(kr + e.kl + j * kstride);
+      const uint64_t* kj = kr + digit_of(j) * kstride;
+      if (j < M)
+        d[j] = up[j < M ? j : 0][k / 2];
+      else
+        d[j] = *reinterpret_cast<const ulonglong2*>(dg + (RAW ? 0 : j * dstride));
+      k0[j] = load_stream2(kj);
+      k1[j] = load_stream2(kj + e.kl);
     }
     const ulonglong2 av = *reinterpret_cast<const ulonglong2*>(a0 ? a0 + (size_t)i * n + s0 : dg);
     uint64_t pre[2][2];
@@ -183,7 +281,7 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
     // Positions s (even) and s + 1 = s ^ 1 land on d(s) and d(s) ^ 1: the
     // automorphism maps brev(s) + N/2 to its image plus N/2 (mod N), so the
     // pair stays an aligned pair, swapped when d(s) is odd (16-byte stores).
-    const uint32_t p = staged(k);
+    const uint32_t p = pair_staged(tid, k);
     const uint32_t s = (uint32_t)wg0 + p;
     uint32_t dst = s;
     if (gi != 1) {
@@ -205,14 +303,18 @@ __device__ __forceinline__ void moddown_pair_body(const uint64_t* __restrict__ y
   }
 }
 
-template <int S, int ND>
+template <int S, int ND, bool RAW>
 __global__ void __launch_bounds__(512)
-    __attribute__((amdgpu_waves_per_eu(ND <= 3 && S >= 7 ? 6 : ND == 4 && S >= 7 ? 8 : 1, 8)))
+    __attribute__((amdgpu_waves_per_eu(RAW                 ? 4
+                                       : ND <= 3 && S >= 7 ? 6
+                                       : ND == 4 && S >= 7 ? 8
+                                                           : 1,
+                                       8)))
     ntt_pass_moddown_pair(const uint64_t* __restrict__ y, const ModConst* __restrict__ mc,
                           const uint64_t* __restrict__ tw_all, uint32_t log_n, uint32_t s_other,
                           const ModDownEpi e) {
   __shared__ uint64_t lds[pair_lds_words<S>()];
-  moddown_pair_body<S, ND>(y, mc, tw_all, log_n, s_other, e, blockIdx.x, blockIdx.y, blockIdx.z,
+  moddown_pair_body<S, ND, RAW>(y, mc, tw_all, log_n, s_other, e, blockIdx.x, blockIdx.y, blockIdx.z,
                            lds);
 }
 
@@ -228,10 +330,11 @@ __global__ void __launch_bounds__(512)
 // N=2^16, 24 limbs).
 // Body for the workgroup at row group bx of P limb t of key switch r, with
 // its tile in lds (pair_lds_words<S>() words).
-template <int S, int ND>
+template <int S, int ND, bool RAW>
 __device__ __forceinline__ void ksk_pair_body(uint64_t* __restrict__ ext, size_t ps,
                                               const ModConst* __restrict__ mc,
-                                              const uint64_t* __restrict__ tw_all, uint32_t log_n,
+                                              const uint64_t* __restrict__ tw_all,
+                                              const uint64_t* __restrict__ tw_fwd, uint32_t log_n,
                                               uint32_t s_other, const ModDownEpi& e, uint32_t bx,
                                               uint32_t r, uint32_t t, uint64_t* lds_base) {
   constexpr int RHO = 2, R = 4, TPL = 1 << (S - RHO), LINES = 512 / TPL;
@@ -247,25 +350,32 @@ __device__ __forceinline__ void ksk_pair_body(uint64_t* __restrict__ ext, size_t
   const size_t wg0 = ((size_t)bx * LINES) << S;
   const uint32_t tau = tid % TPL, line = tid / TPL;
   const uint32_t twbase = (1u << s_other) + bx * LINES + line;
-  auto staged = [&](int k) -> uint32_t {
-    return (tid >> 6) * (64u * R) + (uint32_t)(k >> 1) * 128u + 2 * (tid & 63) + (k & 1);
-  };
+  // RAW: the digits' last forward pass, here and not in a pass of its own.
+  const size_t dstride = (size_t)e.ne * n;
+  ulonglong2 up[RAW ? ND : 1][2];
+  ulonglong2 in[2][2];
+  if constexpr (RAW)
+    finish_digits<S, ND>(
+        lds, in,
+        [&](int j) { return e.digits[r] + j * dstride + (size_t)(e.nq + t) * n + wg0; }, [] {},
+        tw_fwd + (size_t)midx * n * 2, twbase, tau, line, lm, mc[midx].rq, up);
 
   // P-limb key products of both polys into LDS (this wavefront's rows), in
   // (0, 2q) as the first inverse stage accepts them.
   {
-    const size_t dstride = (size_t)e.ne * n, kstride = 2 * e.kl;
+    const size_t kstride = 2 * e.kl;
     const uint64_t qn = e.mc[midx].qinv;
 #pragma unroll
     for (int k = 0; k < R; k += 2) {
-      const uint32_t p = staged(k);
+      const uint32_t p = pair_staged(tid, k);
       const size_t s = wg0 + p;
       const uint64_t* dg = e.digits[r] + (size_t)(e.nq + t) * n + s;
       const uint64_t* kr = e.key[r] + (size_t)midx * n + s;
       ulonglong2 d[ND], k0[ND], k1[ND];
 #pragma unroll
       for (int j = 0; j < ND; ++j) {
-        d[j] = *reinterpret_cast<const ulonglong2*>(dg + j * dstride);
+        d[j] = RAW ? up[RAW ? j : 0][k / 2]
+                   : *reinterpret_cast<const ulonglong2*>(dg + j * dstride);
         k0[j] = load_stream2(kr + j * kstride);
         k1[j] = load_stream2(kr + e.kl + j * kstride);
       }
@@ -340,15 +450,15 @@ __device__ __forceinline__ void ksk_pair_body(uint64_t* __restrict__ ext, size_t
   }
 }
 
-template <int S, int ND>
+template <int S, int ND, bool RAW>
 __global__ void __launch_bounds__(512)
-    __attribute__((amdgpu_waves_per_eu(ND <= 4 ? 8 : 1, 8)))
+    __attribute__((amdgpu_waves_per_eu(RAW ? 4 : ND <= 4 ? 8 : 1, 8)))
     ntt_pass_ksk_pair(uint64_t* __restrict__ ext, size_t ps, const ModConst* __restrict__ mc,
-                      const uint64_t* __restrict__ tw_all, uint32_t log_n, uint32_t s_other,
-                      const ModDownEpi e) {
+                      const uint64_t* __restrict__ tw_all, const uint64_t* __restrict__ tw_fwd,
+                      uint32_t log_n, uint32_t s_other, const ModDownEpi e) {
   __shared__ uint64_t lds[pair_lds_words<S>()];
-  ksk_pair_body<S, ND>(ext, ps, mc, tw_all, log_n, s_other, e, blockIdx.x, blockIdx.y, blockIdx.z,
-                       lds);
+  ksk_pair_body<S, ND, RAW>(ext, ps, mc, tw_all, tw_fwd, log_n, s_other, e, blockIdx.x, blockIdx.y,
+                            blockIdx.z, lds);
 }
 
 template <int S, bool BLK = false>
@@ -363,11 +473,22 @@ void launch_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq, uint32
     constexpr uint32_t pair_lines = 512u >> (S - 2);
     if (npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
       const dim3 grid((1u << s_other) / pair_lines, npoly / 2, nq);
-      switch (epi.nd) {
-#define CASE(D)                                                                                 case D:                                                                                         FHE_LAUNCH(c, name, (ntt_pass_moddown_pair<S, D>), grid, dim3(512), 0, y, c.d_const,                     c.d_tw_fwd, c.log_n, s_other, epi);                                                return;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
-#undef CASE
+#define CASE(D, RAW)                                                                         \
+  case D:                                                                                    \
+    FHE_LAUNCH(c, name, (ntt_pass_moddown_pair<S, D, RAW>), grid, dim3(512), 0, y, c.d_const, \
+               c.d_tw_fwd, c.log_n, s_other, epi);                                           \
+    return;
+      if (epi.raw) {
+        switch (epi.nd) {
+          CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
+        }
+      } else {
+        switch (epi.nd) {
+          CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
+          CASE(6, false) CASE(7, false)
+        }
       }
+#undef CASE
     }
   }
   // The blocked form belongs to the fused ModDown, whose moduli all suit the
@@ -409,15 +530,22 @@ void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other,
     constexpr uint32_t pair_lines = 512u >> (S - 2);
     if (npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
       const dim3 pgrid((1u << s_other) / pair_lines, npoly / 2, c.K);
-      switch (epi.nd) {
-#define CASE(D)                                                                              \
-  case D:                                                                                    \
-    FHE_LAUNCH(c, name, (ntt_pass_ksk_pair<S, D>), pgrid, dim3(512), 0, ext, ps, c.d_const,  \
-               c.d_tw_inv, c.log_n, s_other, epi);                                           \
+#define CASE(D, RAW)                                                                        \
+  case D:                                                                                   \
+    FHE_LAUNCH(c, name, (ntt_pass_ksk_pair<S, D, RAW>), pgrid, dim3(512), 0, ext, ps,       \
+               c.d_const, c.d_tw_inv, c.d_tw_fwd, c.log_n, s_other, epi);                   \
     return;
-        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7)
-#undef CASE
+      if (epi.raw) {
+        switch (epi.nd) {
+          CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
+        }
+      } else {
+        switch (epi.nd) {
+          CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
+          CASE(6, false) CASE(7, false)
+        }
       }
+#undef CASE
     }
   }
   // The blocked form belongs to the fused ModDown, whose moduli all suit the
@@ -458,6 +586,8 @@ void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uin
   if (npoly == 0) return;
   if (npoly > 2 * MAX_KS_BATCH) throw ArgError("ModDown batch too large");
   if (!moddown_fused_ok(c, nq)) throw ArgError("fused ModDown does not apply");
+  if (epi.raw && (epi.nd > RAW_MAX_DIGITS || npoly % 2))
+    throw ArgError("digits without their last pass do not apply");
   const uint32_t s1 = (c.log_n + 1) / 2;
   switch (c.log_n) {
 #define CASE(LN, B)                                                \

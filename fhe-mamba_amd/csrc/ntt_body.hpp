@@ -522,9 +522,10 @@ constexpr int mid_lanes_per_line() {
 // ModUp input: limb blockIdx.z of ciphertext blockIdx.y's c1, read from the
 // caller's polys (the first inverse pass reads them in place of a copy).
 // Each word is read once by the pass, which also stores it as the word of
-// its digit's own limb ([ct][d][ne][N], d = limb / alpha): the digits keep
-// c1's own limbs as they are.
+// its digit's own limb ([ct][d][ne][N], d = limb / alpha) when KEEP: the
+// digits keep c1's own limbs as they are.
 constexpr int MODUP_MAX_CT = 32;
+template <bool KEEP>
 struct SrcLoad {
   static constexpr bool kLoad = true;
   static constexpr bool kPair = false;
@@ -535,7 +536,7 @@ struct SrcLoad {
   __device__ __forceinline__ uint64_t get(size_t g, uint64_t) const {
     const uint32_t ct = blockIdx.y, i = blockIdx.z;
     const uint64_t v = src[ct][(size_t)i * n + g];
-    digits[(((size_t)ct * nd + i / alpha) * ne + i) * n + g] = v;
+    if (KEEP) digits[(((size_t)ct * nd + i / alpha) * ne + i) * n + g] = v;
     return v;
   }
   struct Ops2 {};

@@ -68,9 +68,9 @@ __global__ void __launch_bounds__(max_threads<SINGLE>())
                    const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                    uint32_t log_n, const SrcPtrs src, uint64_t* digits, uint32_t alpha,
                    uint32_t nd, uint32_t ne) {
-  ntt_body<LIM, S, SINGLE, true, RHO_SINGLE, PlainStore, SrcLoad>(
+  ntt_body<LIM, S, SINGLE, true, RHO_SINGLE, PlainStore, SrcLoad<true>>(
       coef, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), 0, PlainStore{},
-      SrcLoad{src.p, 1u << log_n, digits, alpha, nd, ne});
+      SrcLoad<true>{src.p, 1u << log_n, digits, alpha, nd, ne});
 }
 
 template <int LIM, int S>
