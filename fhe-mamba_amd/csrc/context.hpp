@@ -394,8 +394,8 @@ void moddown_mid(Context& c, const uint64_t* ext_p, uint64_t* y, uint32_t npoly,
                  const ConvPlan& pl);
 void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uint32_t nq,
                    const ConvPlan& pl, const ModDownEpi& epi);
-// Rescale of [npoly][nq][N] into out [npoly][nq-1][N] (out != a) in four
-// launches, for ring dimensions 2^13..2^17.
+// Rescale of [npoly][nq][N] into out [npoly][nq-1][N] (out != a) in three
+// launches, or four (rescale.hip has the rule), for ring dimensions 2^13..2^17.
 void rescale_fused(Context& c, uint64_t* out, const uint64_t* a, uint32_t npoly, uint32_t nq);
 // The same for `count` inputs as[r] into outs[r] (each [npoly][nq][N] into
 // [npoly][nq-1][N], no output aliasing any input): up to 16 inputs share
@@ -403,11 +403,10 @@ void rescale_fused(Context& c, uint64_t* out, const uint64_t* a, uint32_t npoly,
 void rescale_fused_many(Context& c, uint64_t* const* outs, const uint64_t* const* as,
                         uint32_t count, uint32_t npoly, uint32_t nq);
 // ModUp of `count` c1 polys (nq limbs each) into digits [count][nd][nq+K][N]
-// in four launches for ring dimensions 2^13..2^17 with every modulus below
-// 2^60: the first inverse pass reading c1 (blocked out), one kernel for the
-// inverse column stages + the conversion of every digit + the forward
-// column stages, the last forward pass, and the copy of each digit's own
-// limbs.
+// in three launches for ring dimensions 2^13..2^17 with every modulus below
+// 2^60: the first inverse pass reading c1 (blocked out) and copying each
+// digit's own limbs, one kernel for the inverse column stages + the conversion
+// of every digit + the forward column stages, and the last forward pass.
 bool modup_fused_ok(const Context& c, uint32_t nq, uint32_t count);
 void modup_fused(Context& c, const uint64_t* const* as, uint32_t count, uint32_t nq,
                  uint64_t* digits);

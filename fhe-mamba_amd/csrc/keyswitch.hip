@@ -167,7 +167,7 @@ __global__ void __launch_bounds__(TPB)
 
 // The key inner product has no kernel of its own: its P limbs feed the
 // first pass of ModDown's inverse NTT and its Q limbs the last pass of the
-// forward NTT (ntt.hip, KskLoad / EpiStore).  Up to MAXD digits.
+// forward NTT (KskLoad / EpiStore).  Up to MAXD digits.
 
 __device__ __forceinline__ uint32_t brev_bits(uint32_t x, uint32_t bits) {
   return __brev(x) >> (32 - bits);
