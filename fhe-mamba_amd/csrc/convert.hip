@@ -88,6 +88,7 @@ struct MidTarget {
   uint32_t qinv_neg;  // -q^-1 mod 2^32
   uint32_t pad_;
 };
+static_assert(sizeof(MidTarget) == 16, "mid_lds_bytes");
 
 // Body for (poly, column) tile `tile` of a workgroup of nw waves (a multiple
 // of 4), with mid_lds_bytes of lds.
@@ -309,8 +310,8 @@ __device__ __forceinline__ void convert_mid_body(const MidArgs& a, const ModCons
 // three workgroups on a CU: 1514 us for the 30-rotation step against 1530 at
 // six and 1593 at eight (spills).
 template <int S1, int S2>
-__global__ void __launch_bounds__(S1 == 9 ? 1024 : 512)
-    __attribute__((amdgpu_waves_per_eu(S1 == 9 ? 4 : S1 == 8 ? 7 : 6, 8)))
+__global__ void __launch_bounds__(64 * mid_max_waves(S1))
+    __attribute__((amdgpu_waves_per_eu(mid_waves_per_simd(S1), 8)))
     k_convert_mid(const MidArgs a, const ModConst* __restrict__ mc,
                   const uint64_t* __restrict__ tw_inv, const uint64_t* __restrict__ tw_fwd) {
   extern __shared__ __align__(16) uint64_t lds_dyn[];
@@ -322,32 +323,13 @@ __global__ void __launch_bounds__(S1 == 9 ? 1024 : 512)
   convert_mid_body<S1, S2>(a, mc, tw_inv, tw_fwd, tile, blockDim.x / 64, lds_dyn);
 }
 
-// LDS of a workgroup of nw waves: target constants (groups of four targets),
-// source lines, lines in flight.
-template <int S1>
-size_t mid_lds_bytes(uint32_t nsrc, uint32_t ndst, uint32_t nw) {
-  const size_t nl = (size_t)nw * (64 / mid_lanes_per_line<S1>());
-  return (size_t)((ndst + 3) / 4) * 4 * sizeof(MidTarget) + (nsrc + nl) * mid_pitch<S1>() * 8;
-}
-
-// Waves per workgroup: 8, so that the source lines of a tile are done in one
-// or two rounds and three workgroups fit a CU (N = 2^16, us a call against 4 /
-// 16 waves: 30 ModDowns at 24 limbs 1553 / 1587 / 1693 for the whole step,
-// one product at 37 limbs 311 / 341 / 324); 16 at N = 2^17, whose lines of 512
-// rows leave one workgroup a CU either way (765 / 817 with 8).
-template <int S1>
-constexpr uint32_t mid_waves() {
-  return S1 == 9 ? 16 : 8;
-}
-
 template <int S1, int S2>
 void launch_mid(Context& c, const char* name, const MidArgs& a, uint32_t npoly,
                 uint32_t max_src, uint32_t max_dst) {
   const uint32_t tiles = npoly << S2;
-  uint32_t nw = mid_waves<S1>();
-  while (nw > 4 && mid_lds_bytes<S1>(max_src, max_dst, nw) > c.lds_per_block) nw /= 2;
+  const uint32_t nw = mid_waves(S1, tiles, max_src, max_dst, c.lds_per_block);
   FHE_LAUNCH(c, name, (k_convert_mid<S1, S2>), dim3(tiles), dim3(64 * nw),
-             (mid_lds_bytes<S1>(max_src, max_dst, nw)), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
+             mid_lds_bytes(S1, max_src, max_dst, nw), a, c.d_const, c.d_tw_inv, c.d_tw_fwd);
 }
 
 // The target order of `pl` must be the one MidPlan describes (checked).
@@ -363,12 +345,8 @@ MidPlan mid_plan(const Context& c, const ConvPlan& pl, uint32_t src_mod0, uint32
 }
 
 bool mid_lds_fits(const Context& c, uint32_t nsrc, uint32_t ndst) {
-  switch (c.log_n) {
-    case 13: case 14: return mid_lds_bytes<7>(nsrc, ndst, 4) <= c.lds_per_block;
-    case 15: case 16: return mid_lds_bytes<8>(nsrc, ndst, 4) <= c.lds_per_block;
-    case 17: return mid_lds_bytes<9>(nsrc, ndst, 4) <= c.lds_per_block;
-    default: return false;
-  }
+  return c.log_n >= 13 && c.log_n <= 17 &&
+         mid_lds_bytes((c.log_n + 1) / 2, nsrc, ndst, 4) <= c.lds_per_block;
 }
 
 // Every modulus of the launch in [2^33, 2^60): the fused kernels' lazy

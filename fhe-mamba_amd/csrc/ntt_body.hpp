@@ -34,6 +34,7 @@
 // table stays hot in L2.
 #pragma once
 
+#include "launch_rules.hpp"
 #include "ops.hpp"
 
 #include <type_traits>
@@ -508,15 +509,14 @@ __device__ __forceinline__ size_t blocked_off(uint32_t b, uint32_t u) {
   return (size_t)(b / BLO) * ((size_t)BLO << S2) + (size_t)u * BLO + (b % BLO);
 }
 
-// LDS words between, and lanes of a wavefront on, the column lines of M = 2^S1
-// rows in kernels that keep whole columns in LDS.
+// Column lines in kernels that keep whole columns in LDS (launch_rules.hpp).
 template <int S1>
 constexpr uint32_t mid_pitch() {
-  return (1u << S1) + (1u << S1) / 16 + 1;
+  return column_pitch(S1);
 }
 template <int S1>
 constexpr int mid_lanes_per_line() {
-  return (1 << S1) / 4 < 64 ? (1 << S1) / 4 : 64;
+  return column_lanes(S1);
 }
 
 // ModUp input: limb blockIdx.z of ciphertext blockIdx.y's c1, read from the

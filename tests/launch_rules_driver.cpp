@@ -1,0 +1,20 @@
+// Host driver for tests/test_launch_rules.py: the launch rules of
+// fhe-mamba_amd/csrc/launch_rules.hpp on lines of
+//   mid S1 TILES NSRC NDST LDS   -> waves, LDS bytes of 4, 8, 16 waves
+#include <cstdio>
+#include <cstring>
+
+#include "launch_rules.hpp"
+
+int main() {
+  char op[16];
+  unsigned a, b, c, d, e;
+  while (scanf("%15s %u %u %u %u %u", op, &a, &b, &c, &d, &e) == 6) {
+    if (!strcmp(op, "mid"))
+      printf("%u %u %u %u\n", fhe::mid_waves(a, b, c, d, e), fhe::mid_lds_bytes(a, c, d, 4),
+             fhe::mid_lds_bytes(a, c, d, 8), fhe::mid_lds_bytes(a, c, d, 16));
+    else
+      return 2;
+  }
+  return 0;
+}

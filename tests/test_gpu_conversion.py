@@ -47,6 +47,38 @@ def test_key_switch_bit_exact(log_n, L, qbits, K, pbits, dnum):
     ctx.close()
 
 
+# (log_n, Q limbs, P limbs, dnum, key switches): the middle kernel's workgroups
+# of 4 waves (lines that fill no more; batches whose 4-wave form keeps at least
+# as many waves on a compute unit), 8 and 16, one batch of targets and several,
+# whole and ragged ones.
+FORMS = [(13, 3, 1, 3, 12), (13, 12, 5, 2, 16), (13, 12, 5, 2, 2), (14, 11, 9, 1, 8),
+         (15, 9, 4, 2, 8), (16, 9, 3, 2, 2), (16, 9, 9, 1, 2), (17, 6, 1, 6, 1), (17, 9, 5, 2, 1),
+         (17, 9, 5, 2, 2), (17, 13, 12, 1, 1)]
+
+
+@pytest.mark.parametrize("log_n,L,K,dnum,count", FORMS)
+def test_middle_kernel_workgroup_forms(log_n, L, K, dnum, count):
+    q = O.ntt_friendly_primes(log_n, 59, L)
+    p = O.ntt_friendly_primes(log_n, 60, K, skip=q)
+    ctx, orc = F.Context(log_n, q, p, dnum, sampling="seeded"), O.Ctx(log_n, q, p, dnum)
+    rng = np.random.default_rng(23)
+    key = residues(rng, list(q) + list(p), (ctx.dnum, 2), ctx.n)
+    dkey = ctx.load_key(key)
+    ct3 = [residues(rng, q, (3,), ctx.n) for _ in range(min(2, count))]
+    want = [orc.relinearize(c, key) for c in ct3]
+    outs = ctx.relinearize_many([ctx.upload(ct3[r % 2]) for r in range(count)], dkey)
+    for r, o in enumerate(outs):
+        assert np.array_equal(o.numpy(), want[r % 2]), r
+    gal = [5, 2 * ctx.n - 1]
+    ct = ctx.upload(ct3[0][:2])
+    want = [orc.rotate(ct3[0][:2], key, g) for g in gal]
+    outs = ctx.rotate_hoisted(ct, ctx.rotation_precompute(ct), [dkey] * count,
+                              [gal[r % 2] for r in range(count)])
+    for r, o in enumerate(outs):
+        assert np.array_equal(o.numpy(), want[r % 2]), r
+    ctx.close()
+
+
 # Q bit sizes, last limb dropped first: primes of one chain, a last prime many
 # times (reduced after its lift) and too many times (four launches) the others.
 RESCALES = [(13, (59, 59, 59)), (14, (60, 45, 59)), (15, (60, 34, 60)), (16, (45, 59)),
