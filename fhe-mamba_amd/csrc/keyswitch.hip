@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "launch_rules.hpp"
 #include "ops.hpp"
 
 namespace fhe {
@@ -423,8 +424,10 @@ void keyswitch_batch(Context& c, const uint64_t* const* digits, uint32_t nq,
 // passes that multiply them by the keys finish them in LDS, which saves
 // writing and re-reading them all (one rotation at N=2^16, us: 24 limbs, 3
 // digits 127 -> 114; N=2^17 multiplication of 41 limbs, 4 digits 735 -> 642).
-// Up to RAW_MAX_DIGITS digits, what two workgroups a CU have registers for.
-// Digits that several key switches share are finished once, by modup_batch.
+// Up to RAW_MAX_DIGITS digits, what two workgroups a CU have registers for,
+// and not for the smallest switches of three or more
+// (finish_digits_in_moddown).  Digits that several key switches share are
+// finished once, by modup_batch.
 static void switch_each(Context& c, const uint64_t* const* srcs, uint32_t nq,
                         const uint64_t* const* keys, uint32_t count, const KeySwitchOut* outs,
                         uint64_t* dig) {
@@ -432,7 +435,8 @@ static void switch_each(Context& c, const uint64_t* const* srcs, uint32_t nq,
   const size_t ct_words = (size_t)nd * (nq + c.K) * c.n;
   std::vector<const uint64_t*> dg(count);
   for (uint32_t r = 0; r < count; ++r) dg[r] = dig + r * ct_words;
-  const bool raw = nd <= RAW_MAX_DIGITS && modup_fused_ok(c, nq, count) && moddown_fused_ok(c, nq);
+  const bool raw = nd <= RAW_MAX_DIGITS && finish_digits_in_moddown(nd, nq + c.K, c.n, count) &&
+                   modup_fused_ok(c, nq, count) && moddown_fused_ok(c, nq);
   if (raw)
     modup_raw(c, srcs, count, nq, dig);
   else

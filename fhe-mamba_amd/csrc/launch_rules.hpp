@@ -58,4 +58,19 @@ inline uint32_t mid_waves(uint32_t s1, uint32_t tiles, uint32_t nsrc, uint32_t n
   return best;
 }
 
+// ---- Digits that one key switch uses ----
+// Whether their last block stages run inside ModDown's passes (modup_raw), for
+// `count` key switches of nd digits of `limbs` limbs in one launch set.  That
+// saves a pass over the digits, and makes them in turn, two at a time, in
+// ModDown's workgroups: with three digits or more that chain costs more than
+// the pass while the digits are small.  One rotation, us, in a pass of their
+// own / inside: 4 digits of 5 limbs at N=2^13 35.0 / 38.5 (1.2 MiB), at N=2^14
+// 38.1 / 42.1 (2.5), at N=2^15 44.5 / 46.8 (5); 4 digits of 20 limbs at N=2^13
+// 45.5 / 44.5 (5), 3 of 32 47.9 / 46.0 (6), at N=2^15 3 of 20 61.7 / 57.0 (15).
+// With two digits this is at most 2.5% behind and up to 15% ahead, with one 3
+// to 12% ahead, at any size.
+constexpr bool finish_digits_in_moddown(uint32_t nd, uint32_t limbs, uint32_t n, uint32_t count) {
+  return nd <= 2 || (uint64_t)count * nd * limbs * n * 8 > (5u << 20);
+}
+
 }  // namespace fhe

@@ -1,6 +1,7 @@
 // Host driver for tests/test_launch_rules.py: the launch rules of
 // fhe-mamba_amd/csrc/launch_rules.hpp on lines of
 //   mid S1 TILES NSRC NDST LDS   -> waves, LDS bytes of 4, 8, 16 waves
+//   digits ND LIMBS N COUNT 0    -> 1 if finished inside ModDown
 #include <cstdio>
 #include <cstring>
 
@@ -13,6 +14,8 @@ int main() {
     if (!strcmp(op, "mid"))
       printf("%u %u %u %u\n", fhe::mid_waves(a, b, c, d, e), fhe::mid_lds_bytes(a, c, d, 4),
              fhe::mid_lds_bytes(a, c, d, 8), fhe::mid_lds_bytes(a, c, d, 16));
+    else if (!strcmp(op, "digits"))
+      printf("%d\n", (int)fhe::finish_digits_in_moddown(a, b, c, d));
     else
       return 2;
   }

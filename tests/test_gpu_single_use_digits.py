@@ -42,3 +42,28 @@ def test_single_use_digits(log_n, L, K, dnum):
             assert np.array_equal(ctx.relinearize(ctx.upload(ct3), dkeys[1]).numpy(),
                                   orc.relinearize(ct3, keys[1]))
     ctx.close()
+
+
+@pytest.mark.parametrize("log_n,L,K,dnum,count,inside", [
+    (13, 3, 1, 3, 1, False), (13, 4, 1, 4, 2, False), (14, 7, 2, 4, 1, False),
+    (15, 4, 1, 4, 1, False), (13, 2, 1, 2, 1, True), (13, 4, 1, 4, 32, True),
+    (16, 3, 1, 3, 1, True)])
+def test_small_switches_keep_the_digits_pass(log_n, L, K, dnum, count, inside):
+    """Three or four digits of 5 MiB or less in all are finished by a pass of
+    their own, whose chain is shorter; the others inside ModDown."""
+    q = O.ntt_friendly_primes(log_n, 58, L)
+    p = O.ntt_friendly_primes(log_n, 59, K, skip=q)
+    ctx, orc = F.Context(log_n, q, p, dnum, sampling="seeded"), O.Ctx(log_n, q, p, dnum)
+    rng = np.random.default_rng(5)
+    key = residues(rng, list(q) + list(p), (ctx.dnum, 2), ctx.n)
+    dkey = ctx.load_key(key)
+    ct = residues(rng, q, (2,), ctx.n)
+    cts = [ctx.upload(ct) for _ in range(count)]
+    ctx.profile_begin()
+    outs = ctx.rotate_many(cts, [dkey] * count, [5] * count)
+    kernels = ctx.profile_end()
+    want = orc.rotate(ct, key, 5)
+    for o in outs:
+        assert np.array_equal(o.numpy(), want)
+    assert ("ntt_fwd_blocks_modup" in kernels) is not inside, kernels
+    ctx.close()

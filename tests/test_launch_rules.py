@@ -75,3 +75,13 @@ def test_middle_kernel_waves_with_little_lds(rules):
     for (s1, _, nsrc, ndst, _), (nw, *lds) in zip(shapes, rules("mid", shapes)):
         if lds[0] <= 65536:
             assert lds[{4: 0, 8: 1, 16: 2}[nw]] <= 65536, (s1, nsrc, ndst, nw)
+
+
+def test_digits_finished_in_moddown(rules):
+    """One and two digits always, more only above 5 MiB of digits, as measured."""
+    want = {(1, 2, 1 << 13, 1): 1, (2, 3, 1 << 13, 1): 1, (3, 4, 1 << 13, 1): 0,
+            (4, 5, 1 << 13, 1): 0, (4, 5, 1 << 14, 2): 0, (4, 5, 1 << 15, 1): 0,
+            (3, 32, 1 << 13, 1): 1, (3, 20, 1 << 15, 1): 1, (4, 5, 1 << 13, 32): 1,
+            (3, 32, 1 << 16, 1): 1, (4, 53, 1 << 17, 32): 1}
+    got = rules("digits", [(*s, 0) for s in want])
+    assert {s: r[0] for s, r in zip(want, got)} == want
