@@ -73,4 +73,41 @@ constexpr bool finish_digits_in_moddown(uint32_t nd, uint32_t limbs, uint32_t n,
   return nd <= 2 || (uint64_t)count * nd * limbs * n * 8 > (5u << 20);
 }
 
+// ---- Rescale, N = 2^13 .. 2^17 ----
+// `tiles` columns of the last limb lifted into l other limbs.  Whether one
+// kernel per column does it (k_rescale_mid, three launches) and not two column
+// passes (four).  The column kernel is ahead except in batches of rings with 128
+// rows a column, where its waves, of two lines each, wait for the one that has
+// the last limb; the line lies where the intermediate (tiles l KiB) outgrows the
+// L2s (32 MiB).  s1 = 7, us, as three launches of 4-wave workgroups / as four:
+// 1536 tiles of 19 limbs 44.1 / 46.5 (29 MiB), 4096 of 8 48.7 / 47.0 (32), 2048
+// of 19 53.1 / 52.9 (38), of 39 101 / 90, 4096 of 23 122 / 116.  s1 = 8: 8192 of
+// 29 limbs 521 / 606; s1 = 9: 8192 of 44 limbs 1685 / 2278.
+constexpr bool rescale_by_columns(uint32_t s1, uint32_t tiles, uint32_t l) {
+  return s1 > 7 || tiles <= 1024 || (uint64_t)tiles * l <= 32768;
+}
+// Waves of the column kernel's workgroup.  us at 4 / 8 / 16 waves:
+//  - no more than the lines fill: 4 limbs, 32 polys, N=2^16 86 / 91 / 109, and
+//    one limb, 2 / 4 / 8 waves: N=2^14 22.0 / 23.6 / 27.0, N=2^17 78 / 84 / 118;
+//  - 16 where a launch leaves half the chip's wave slots free at 8, one
+//    ciphertext at N=2^16: 12 limbs 25.4 / 24.6 / 24.5, 29 limbs 43.2 / 42.6 /
+//    41.5; N=2^15: 44 limbs 40.1 / 35.8 / 34.6; N=2^13 44 limbs 26.9 / 23.4 /
+//    22.5.  Not with 512 rows a column, whose lines hold 8 rows a lane: N=2^17
+//    16 limbs 52.1 / 51.2 / 54.1, 44 limbs 121.8 / 119.4 / 120.7; nor above 512
+//    tiles: 3 polys at N=2^16, 29 limbs 54.6 / 53.7 / 53.8, 8 polys at N=2^14,
+//    44 limbs 57.5 / 57.8 / 63.3;
+//  - 4 in batches with 128 rows a column (two lines a wave): 20 polys at
+//    N=2^13, 19 limbs 38.1 / 41.9 / 43.5; 8 else (32 polys, 44 limbs, N=2^16 795
+//    / 792 / 814).
+constexpr uint32_t rescale_waves(uint32_t s1, uint32_t tiles, uint32_t l) {
+  const uint32_t rounds = (l + column_lines(s1) - 1) / column_lines(s1);  // of one wave
+  if (rounds <= 2) return 2;
+  if (rounds <= 4 || (s1 == 7 && tiles > 1024)) return 4;
+  return rounds > 8 && tiles <= 512 && s1 < 9 ? 16 : 8;
+}
+// LDS: the last limb's line and a line for each in flight.
+constexpr uint32_t rescale_lds_bytes(uint32_t s1, uint32_t nw) {
+  return (1 + nw * column_lines(s1)) * column_pitch(s1) * 8;
+}
+
 }  // namespace fhe

@@ -1,4 +1,4 @@
-// Rescale as four passes of ntt_body.hpp.
+// Rescale in three launches, or four passes of ntt_body.hpp.
 #include "rescale_parts.hpp"
 
 namespace fhe {
@@ -13,8 +13,8 @@ namespace {
 // kernel per column does the inverse column stages of the last limb, its
 // centred lift and the forward column stages of every other limb
 // (k_rescale_mid, blocked layout on both sides): three launches.  For other
-// moduli an inverse column pass and a forward one that lifts as it loads
-// (LiftLoad): four.
+// moduli, and where rescale_by_columns says so, an inverse column pass and a
+// forward one that lifts as it loads (LiftLoad): four.
 
 // One workgroup per (launch poly, column) tile, nw waves, LPW column lines a
 // wave.  The first line's wave takes the last limb to centred coefficients v
@@ -140,7 +140,7 @@ __device__ __forceinline__ void rescale_mid_body(
 }
 
 template <int S1, int S2>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(S1 == 9 ? 512 : 1024)
     __attribute__((amdgpu_waves_per_eu(S1 == 9 ? 4 : 8, 8)))
     k_rescale_mid(const uint64_t* __restrict__ last, uint64_t* __restrict__ t,
                   const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_inv,
@@ -198,18 +198,6 @@ __global__ void __launch_bounds__(256)
 
 }  // namespace
 
-template <int S1>
-static size_t rescale_mid_lds(uint32_t nw) {
-  return (size_t)(1 + nw * (64 / mid_lanes_per_line<S1>())) * mid_pitch<S1>() * 8;
-}
-template <int S1>
-static uint32_t rescale_waves(uint32_t tiles, uint32_t l) {
-  // One ciphertext (512 tiles at N = 2^16) leaves half of the chip's wave slots
-  // idle at 8 waves: 42.0 against 43.0 us a rescale at 30 limbs.
-  const uint32_t lines = (l + 64 / mid_lanes_per_line<S1>() - 1) / (64 / mid_lanes_per_line<S1>());
-  return lines <= 4 ? 4 : lines > 8 && tiles <= 1024 ? 16 : 8;
-}
-
 static void rescale_launch(Context& c, uint64_t* const* outs, const uint64_t* const* as,
                            uint32_t count, uint32_t npoly, uint32_t nq);
 
@@ -259,11 +247,11 @@ static void rescale_launch(Context& c, uint64_t* const* outs, const uint64_t* co
                  dim3(tb, np, l), dim3(256), 0, t.p, (size_t)l * n, c.d_const, c.d_tw_fwd,    \
                  c.log_n, s1, ptrs, c.d_rescale, l, c.L, npoly);                              \
     };                                                                                        \
-    if (mid) {                                                                                \
-      const uint32_t nw = rescale_waves<A>(np << B, l);                                       \
+    if (mid && rescale_by_columns(A, np << B, l)) {                                           \
+      const uint32_t nw = rescale_waves(A, np << B, l);                                       \
       in(std::integral_constant<int, 16>{});                                                  \
       FHE_LAUNCH(c, "k_rescale_mid", (k_rescale_mid<A, B>), dim3(np << B), dim3(64 * nw),     \
-                 rescale_mid_lds<A>(nw), last.p, t.p, c.d_const, c.d_tw_inv, c.d_tw_fwd,      \
+                 rescale_lds_bytes(A, nw), last.p, t.p, c.d_const, c.d_tw_inv, c.d_tw_fwd,    \
                  c.d_rescale, l, c.L);                                                        \
       out(std::integral_constant<int, 16>{});                                                 \
       return;                                                                                 \

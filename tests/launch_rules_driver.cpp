@@ -2,6 +2,7 @@
 // fhe-mamba_amd/csrc/launch_rules.hpp on lines of
 //   mid S1 TILES NSRC NDST LDS   -> waves, LDS bytes of 4, 8, 16 waves
 //   digits ND LIMBS N COUNT 0    -> 1 if finished inside ModDown
+//   rescale S1 TILES L 0 0       -> 1 if by the column kernel, its waves
 #include <cstdio>
 #include <cstring>
 
@@ -16,6 +17,8 @@ int main() {
              fhe::mid_lds_bytes(a, c, d, 8), fhe::mid_lds_bytes(a, c, d, 16));
     else if (!strcmp(op, "digits"))
       printf("%d\n", (int)fhe::finish_digits_in_moddown(a, b, c, d));
+    else if (!strcmp(op, "rescale"))
+      printf("%d %u\n", (int)fhe::rescale_by_columns(a, b, c), fhe::rescale_waves(a, b, c));
     else
       return 2;
   }

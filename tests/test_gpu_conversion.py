@@ -100,3 +100,27 @@ def test_rescale_moduli(log_n, bits):
     for a in [residues(rng, q, (2,), ctx.n), pats[1:3], np.stack([half, pats[3]])]:
         assert np.array_equal(ctx.rescale(ctx.upload(a)).numpy(), orc.rescale(a))
     ctx.close()
+
+
+# (log_n, limbs, polys, ciphertexts, column kernel): batches on both sides of
+# the line between three launches and four, and rings that have no such line.
+BATCHES = [(14, 2, 2, 16, True), (17, 3, 1, 2, True), (13, 20, 2, 10, True), (13, 20, 2, 16, False), (14, 9, 2, 16, True),
+           (14, 10, 2, 16, False), (14, 18, 2, 8, False), (14, 18, 2, 4, True),
+           (15, 10, 2, 16, True), (16, 10, 2, 16, True)]
+
+
+@pytest.mark.parametrize("log_n,nq,npoly,count,columns", BATCHES)
+def test_rescale_batches(log_n, nq, npoly, count, columns):
+    q = O.ntt_friendly_primes(log_n, 59, nq)
+    ctx, orc = F.Context(log_n, q, [], 1, sampling="seeded"), O.Ctx(log_n, q, [], 1)
+    rng = np.random.default_rng(29)
+    xs = [residues(rng, q, (npoly,), ctx.n) for _ in range(2)]
+    want = [orc.rescale(x) for x in xs]
+    dev = [ctx.upload(xs[r % 2]) for r in range(count)]
+    ctx.profile_begin()
+    outs = ctx.rescale_many(dev)
+    kernels = ctx.profile_end()
+    for r, o in enumerate(outs):
+        assert np.array_equal(o.numpy(), want[r % 2]), r
+    assert ("k_rescale_mid" in kernels) is columns, kernels
+    ctx.close()

@@ -85,3 +85,21 @@ def test_digits_finished_in_moddown(rules):
             (3, 32, 1 << 16, 1): 1, (4, 53, 1 << 17, 32): 1}
     got = rules("digits", [(*s, 0) for s in want])
     assert {s: r[0] for s, r in zip(want, got)} == want
+
+
+def test_rescale_route(rules):
+    """The column kernel but for batches of 128-row columns whose intermediate
+    is over 32 MiB; its waves no more than the lines fill, 16 for up to 512 tiles
+    below 512 rows, as measured."""
+    shapes = [(s1, tiles, l, 0, 0) for s1 in (7, 8, 9)
+              for tiles in (64, 128, 512, 768, 1024, 1280, 2048, 4096, 16384)
+              for l in (1, 2, 4, 8, 9, 12, 16, 17, 19, 29, 44, 63)]
+    for (s1, tiles, l, _, _), (columns, nw) in zip(shapes, rules("rescale", shapes)):
+        what = (s1, tiles, l, columns, nw)
+        assert columns == (s1 > 7 or tiles <= 1024 or tiles * l <= 32 * 1024), what
+        assert nw in (2, 4, 8, 16) and (nw == 2 or l > nw // 2 * lines_per_wave(s1)), what
+        assert nw < 16 or (tiles <= 512 and s1 < 9), what
+    want = {(7, 4096, 1): 2, (9, 4096, 1): 2, (8, 8192, 4): 4, (8, 512, 29): 16, (7, 128, 44): 16, (9, 512, 44): 8,
+            (8, 768, 29): 8, (7, 1024, 44): 8, (7, 1280, 19): 4, (8, 8192, 44): 8}
+    got = rules("rescale", [(*s, 0, 0) for s in want])
+    assert {s: r[1] for s, r in zip(want, got)} == want
