@@ -105,9 +105,13 @@ constexpr uint32_t rescale_waves(uint32_t s1, uint32_t tiles, uint32_t l) {
   if (rounds <= 4 || (s1 == 7 && tiles > 1024)) return 4;
   return rounds > 8 && tiles <= 512 && s1 < 9 ? 16 : 8;
 }
-// LDS: the last limb's line and a line for each in flight.
+// LDS: the last limb's line and one for each in flight, in the 64 KB that any
+// device gives a workgroup for every form above.
 constexpr uint32_t rescale_lds_bytes(uint32_t s1, uint32_t nw) {
   return (1 + nw * column_lines(s1)) * column_pitch(s1) * 8;
 }
+static_assert(rescale_lds_bytes(7, 16) <= 65536 && rescale_lds_bytes(8, 16) <= 65536 &&
+                  rescale_lds_bytes(9, 8) <= 65536,
+              "rescale workgroups");
 
 }  // namespace fhe

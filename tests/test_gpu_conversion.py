@@ -124,3 +124,19 @@ def test_rescale_batches(log_n, nq, npoly, count, columns):
         assert np.array_equal(o.numpy(), want[r % 2]), r
     assert ("k_rescale_mid" in kernels) is columns, kernels
     ctx.close()
+
+
+# One ciphertext: 16 waves (more than 8 rounds of lines) at each column length
+# that has that form, 8 at N=2^17, limb counts that do and do not fill a round.
+SINGLES = [(13, 19), (13, 20), (14, 19), (14, 34), (15, 12), (15, 18), (16, 12), (17, 20),
+           (17, 41)]
+
+
+@pytest.mark.parametrize("log_n,nq", SINGLES)
+def test_rescale_of_one_ciphertext(log_n, nq):
+    q = O.ntt_friendly_primes(log_n, 59, nq)
+    ctx, orc = F.Context(log_n, q, [], 1, sampling="seeded"), O.Ctx(log_n, q, [], 1)
+    for npoly in (1, 2):
+        x = residues(np.random.default_rng(31), q, (npoly,), ctx.n)
+        assert np.array_equal(ctx.rescale(ctx.upload(x)).numpy(), orc.rescale(x)), npoly
+    ctx.close()
