@@ -51,7 +51,7 @@ struct ModConst {
   uint64_t wninv_sh;
   uint64_t r2;         // 2^128 mod q (to Montgomery form via redc)
   // 2^64 - q and 2^64 - 4q, read from memory so that the compiler keeps
-  // additions of them (shoup_lazy4n, lazy_sub) instead of folding them back
+  // additions of them (shoup_acc, lazy_sub) instead of folding them back
   // into borrow-chain subtractions.
   uint64_t neg_q, neg_q4;
   uint64_t qinv;       // q^-1 mod 2^64 (redc_lazy)

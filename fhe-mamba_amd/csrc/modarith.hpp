@@ -26,19 +26,6 @@ FHE_HD uint64_t shoup_lazy(uint64_t a, uint64_t w, uint64_t wp, uint64_t q) {
   return a * w - mulhi64(a, wp) * q;
 }
 
-// Shoup product with an approximate quotient: the low partial product
-// a_lo * wp_lo and the carries of the two middle products are dropped, so
-// the quotient is low by 0, 1 or 2 and the result a*w mod q plus 0..3 q lies
-// in [0, 4q) for any a < 2^64 (three 32x32 multiplies for the quotient
-// instead of four and the carry chain).  Needs 4q < 2^64.
-FHE_HD uint64_t shoup_lazy4(uint64_t a, uint64_t w, uint64_t wp, uint64_t q) {
-  const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
-  const uint32_t p0 = (uint32_t)wp, p1 = (uint32_t)(wp >> 32);
-  const uint64_t qt = (uint64_t)a1 * p1 + (((uint64_t)a0 * p1) >> 32) +
-                      (((uint64_t)a1 * p0) >> 32);
-  return a * w - qt * q;
-}
-
 // Keeps a value in vector registers in the form it has here.  The compiler
 // narrows a 64-bit sum of products whose low word alone is used to separate
 // 32-bit multiplies and adds; gfx950 issues v_mad_u64_u32 at the rate of
@@ -56,15 +43,18 @@ FHE_HD uint32_t keep32(uint32_t v) {
   return v;
 }
 
-// x + T mod 2^64, T = a*w mod q plus 0..3 q in [0, 4q) for any a < 2^64:
-// shoup_lazy4's quotient, the remainder accumulated against qneg = 2^64 - q
-// (a*w - qt*q = a*w + qt*qneg mod 2^64).  Both the addend x and the four
-// products of the high word ride in v_mad_u64_u32 accumulations: 11 VALU
-// instructions with no borrow chain (measured in registers, the forward
-// butterfly built on it takes 16.7 issue cycles against 20.5 for adding x to
-// a finished product with 32-bit multiplies in the high word).  `one` is 1,
-// read from memory where it matters: v_mad_u64_u32(h, one, x) adds a 32-bit h
-// to a 64-bit x without first zero-extending it into a register pair.
+// x + T mod 2^64 for the Shoup product T = a*w mod q plus 0..3 q in [0, 4q),
+// any a < 2^64 (4q < 2^64).  The quotient drops the low partial product a_lo
+// wp_lo and the carries of the two middle products, so it is low by 0, 1 or 2
+// (three 32x32 multiplies and no carry chain); the remainder is accumulated
+// against qneg = 2^64 - q (a*w - qt*q = a*w + qt*qneg mod 2^64).  Both the
+// addend x and the four products of the high word ride in v_mad_u64_u32
+// accumulations: 11 VALU instructions with no borrow chain (measured in
+// registers, the forward butterfly built on it takes 16.7 issue cycles against
+// 20.5 for adding x to a finished product with 32-bit multiplies in the high
+// word).  `one` is 1, read from memory where it matters: v_mad_u64_u32(h, one,
+// x) adds a 32-bit h to a 64-bit x without first zero-extending it into a
+// register pair.
 FHE_HD uint64_t shoup_acc(uint64_t x, uint64_t a, uint64_t w, uint64_t wp, uint64_t qneg,
                            uint32_t one = 1) {
   const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32);
@@ -81,11 +71,6 @@ FHE_HD uint64_t shoup_acc(uint64_t x, uint64_t a, uint64_t w, uint64_t wp, uint6
   h += (uint64_t)t1 * n0;
   const uint32_t hi = keep32((uint32_t)(lo >> 32) + (uint32_t)keep64(h));
   return ((uint64_t)hi << 32) | (uint32_t)lo;
-}
-
-// a*w mod q plus 0..3 q, in [0, 4q) for any a < 2^64.
-FHE_HD uint64_t shoup_lazy4n(uint64_t a, uint64_t w, uint64_t wp, uint64_t qneg) {
-  return shoup_acc(0, a, w, wp, qneg);
 }
 
 // x >= m ? x - m : x for nm = 2^64 - m, m <= 2^63 and x - m < 2^63 when

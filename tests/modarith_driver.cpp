@@ -1,8 +1,7 @@
 // Host driver for tests/test_modarith_bounds.py: evaluates the modular
-// helpers of fhe-mamba_amd/csrc/modarith.hpp (compiled for the host, the
-// same source the kernels use) and the butterflies the NTT kernels build
-// from them, on records of little-endian uint64 read from stdin; writes
-// one or two uint64 per record to stdout.
+// helpers and the NTT butterflies of fhe-mamba_amd/csrc/modarith.hpp (compiled
+// for the host, the same source the kernels use) on records of little-endian
+// uint64 read from stdin; writes one or two uint64 per record to stdout.
 //
 //   modarith_driver OP < records > results
 #include <cmath>
@@ -29,10 +28,10 @@ int main(int argc, char** argv) {
   struct Op {
     const char* name;
     int in, out;
-  } ops[] = {{"shoup_lazy", 2, 1},   {"shoup_lazy4", 2, 1}, {"shoup_lazy4n", 2, 1},
-             {"lazy_sub", 2, 1},     {"redc", 2, 1},        {"redc_lazy", 2, 1},
-             {"reduce_est", 1, 1},   {"fwd", 3, 2},         {"inv", 3, 2},
-             {"fwd_alt_even", 3, 2}, {"fwd_alt_odd", 3, 2}};
+  } ops[] = {{"shoup_lazy", 2, 1}, {"shoup_acc", 3, 1},    {"lazy_sub", 2, 1},
+             {"redc", 2, 1},       {"redc_lazy", 2, 1},    {"reduce_est", 1, 1},
+             {"fwd", 3, 2},        {"inv", 3, 2},          {"fwd_alt_even", 3, 2},
+             {"fwd_alt_odd", 3, 2}};
   int nin = 0, nout = 0;
   for (const Op& o : ops)
     if (!strcmp(o.name, op)) nin = o.in, nout = o.out;
@@ -41,14 +40,12 @@ int main(int argc, char** argv) {
   std::vector<uint64_t> rec(nin + 1);
   uint64_t res[2];
   while (fread(rec.data(), 8, nin + 1, stdin) == (size_t)(nin + 1)) {
-    const uint64_t q = rec[0], qneg = 0 - q, q4 = 4 * q, q4neg = 0 - 4 * q, q8neg = 0 - 8 * q;
+    const uint64_t q = rec[0], qneg = 0 - q;
     const uint64_t* a = rec.data() + 1;
     if (!strcmp(op, "shoup_lazy")) {
       res[0] = shoup_lazy(a[0], a[1], host_shoup(a[1], q), q);
-    } else if (!strcmp(op, "shoup_lazy4")) {
-      res[0] = shoup_lazy4(a[0], a[1], host_shoup(a[1], q), q);
-    } else if (!strcmp(op, "shoup_lazy4n")) {
-      res[0] = shoup_lazy4n(a[0], a[1], host_shoup(a[1], q), qneg);
+    } else if (!strcmp(op, "shoup_acc")) {
+      res[0] = shoup_acc(a[0], a[1], a[2], host_shoup(a[2], q), qneg);
     } else if (!strcmp(op, "lazy_sub")) {
       res[0] = lazy_sub(a[0], 0 - a[1]);  // x >= m ? x - m : x with m = a[1]
     } else if (!strcmp(op, "redc")) {
@@ -58,21 +55,20 @@ int main(int argc, char** argv) {
     } else if (!strcmp(op, "reduce_est")) {
       res[0] = reduce_est(a[0], qneg, rq_of(q));
     } else {
-      // Butterflies of the NTT kernels on (x, y, w): forward Cooley-Tukey
-      // with X brought below 4q (plain) or 8q (the even stages of the
-      // alternating range) or taken as is (its odd stages); inverse
-      // Gentleman-Sande with the sum brought below 4q.
-      const uint64_t x = a[0], y = a[1], w = a[2], wp = host_shoup(w, q);
+      // The kernels' butterflies on (x, y, w): Cooley-Tukey in the narrow range
+      // (LIM = 8, X brought below 4q) and on the even and odd stages of the wide
+      // one (LIM = 16: X brought below 8q, or taken as it is), Gentleman-Sande
+      // in the narrow range from inputs below 4q.
+      const bool wide = !strncmp(op, "fwd_alt", 7);
+      const LazyMod m{4 * q, 8 * q, qneg, 0 - (wide ? 8 : 4) * q, 1};
+      const uint64_t w = a[2], wp = host_shoup(w, q);
+      res[0] = a[0];
+      res[1] = a[1];
       if (!strcmp(op, "inv")) {
-        res[1] = shoup_lazy4n(x + q4 - y, w, wp, qneg);
-        res[0] = lazy_sub(x + y, q4neg);
+        int bx = 4, by = 4;
+        inv_butterfly(res[0], res[1], w, wp, m, 8, bx, by);
       } else {
-        const uint64_t X = !strcmp(op, "fwd")            ? lazy_sub(x, q4neg)
-                           : !strcmp(op, "fwd_alt_even") ? lazy_sub(x, q8neg)
-                                                         : x;
-        const uint64_t T = shoup_lazy4n(y, w, wp, qneg);
-        res[0] = X + T;
-        res[1] = X + q4 - T;
+        fwd_butterfly(res[0], res[1], w, wp, m, strcmp(op, "fwd_alt_odd") != 0);
       }
     }
     fwrite(res, 8, nout, stdout);

@@ -1,9 +1,8 @@
 """The lazy-reduction bounds that bit-exactness rests on, checked on the CPU.
 
 fhe-mamba_amd/csrc/modarith.hpp is compiled for the host (tests/
-modarith_driver.cpp: the kernels' own helpers, and the NTT butterflies
-composed from them as the kernels compose them) and every result is
-checked with unbounded integers: the congruence and the stated output range,
+modarith_driver.cpp: the kernels' own helpers and NTT butterflies) and every
+result is checked with unbounded integers: the congruence and the stated output range,
 on random inputs across the stated input range and on inputs at its edges
 (0, the largest allowed value, both ends of the modulus range).  This is the
 method of the reference's experiments/ntt_lazy/check_arithmetic.py (integer
@@ -59,10 +58,11 @@ def edge_and_random(rng, hi, edges):
     return vals + [rng.randrange(hi) for _ in range(N_RANDOM)]
 
 
-@pytest.mark.parametrize("op,bound", [("shoup_lazy", 2), ("shoup_lazy4", 4), ("shoup_lazy4n", 4)])
+@pytest.mark.parametrize("op,bound", [("shoup_lazy", 2), ("shoup_acc", 4)])
 def test_shoup_products(driver, op, bound):
     """a * w mod q for any 64-bit a and w < q: [0, 2q) exact quotient,
-    [0, 4q) approximate quotient (three 32x32 partial products)."""
+    [0, 4q) approximate quotient (three 32x32 partial products), which is
+    added to any 64-bit x modulo 2^64."""
     rng = random.Random(11)
     recs = []
     for q in Q_PLAIN:
@@ -70,11 +70,14 @@ def test_shoup_products(driver, op, bound):
         a_vals = edge_and_random(rng, R64, [0, 1, q - 1, q, 4 * q - 1, 8 * q - 1, M64,
                                             M64 - q, 1 << 63, (1 << 32) - 1, 1 << 32])
         for i, a in enumerate(a_vals):
-            recs.append((q, a, ws[i % len(ws)]))
+            x = [0, M64, rng.randrange(R64)][i % 3]
+            recs.append((q, x, a, ws[i % len(ws)]) if op == "shoup_acc"
+                        else (q, a, ws[i % len(ws)]))
     out = run(driver, op, recs, 1)
-    for (q, a, w), (r,) in zip(recs, out):
-        assert 0 <= r < bound * q, (op, q, a, w, r)
-        assert r % q == a * w % q, (op, q, a, w, r)
+    for (q, *x, a, w), (r,) in zip(recs, out):
+        t = (r - x[0]) % R64 if x else r
+        assert 0 <= t < bound * q, (op, q, x, a, w, r)
+        assert t % q == a * w % q, (op, q, x, a, w, r)
 
 
 def test_lazy_sub(driver):
@@ -172,7 +175,7 @@ def test_inverse_butterfly(driver):
 
 
 def test_alternating_forward_range(driver):
-    """The fused ModDown's alternating range (q < 2^60): a stage that first
+    """The wide range's alternating stages (q < 2^60): a stage that first
     brings X below 8q takes inputs below 16q and leaves them below 12q; the
     next stage adds without reducing and leaves them below 16q; the sum the
     epilogue reduces (last stage < 12q, key sum < 2q, addend < q) is below
