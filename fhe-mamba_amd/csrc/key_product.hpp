@@ -24,96 +24,31 @@ __device__ __forceinline__ ulonglong2 load_stream2(const uint64_t* p) {
 }
 
 // Key inner product sum_j d_j k_j reduced once by REDC (keys in Montgomery
-// form).  SPLIT (every modulus below 2^60, at most 7 digits): operands split
-// at bit 30 and accumulated carry-free in three 64-bit sums with
-// v_mad_u64_u32, T = a0 + a1 2^30 + a2 2^60; otherwise 128-bit products.
-template <int ND, bool SPLIT>
+// form).
+template <int ND>
 __device__ __forceinline__ uint64_t key_dot(const uint64_t* dg, size_t dstride, const uint64_t* kr,
                                             size_t kstride, uint32_t nd_rt, uint64_t q,
                                             uint64_t qinv_neg) {
-  if constexpr (SPLIT && ND > 0 && ND <= 7) {
-    constexpr uint32_t M30 = (1u << 30) - 1;
-    uint64_t a0 = 0, a1 = 0, a2 = 0;
+  Acc128 acc;
+  if (ND > 0) {
 #pragma unroll
-    for (int j = 0; j < ND; ++j) {
-      const uint64_t d = dg[j * dstride], k = load_stream(kr + j * kstride);
-      const uint32_t dl = (uint32_t)d & M30, dh = (uint32_t)(d >> 30);
-      const uint32_t kl = (uint32_t)k & M30, kh = (uint32_t)(k >> 30);
-      a0 += (uint64_t)dl * kl;
-      a1 += (uint64_t)dl * kh;
-      a1 += (uint64_t)dh * kl;
-      a2 += (uint64_t)dh * kh;
-    }
-    const uint64_t m1 = a1 << 30, m2 = a2 << 60;
-    const uint64_t lo = a0 + m1;
-    uint64_t hi = (a1 >> 34) + (a2 >> 4) + (lo < m1);
-    const uint64_t lo2 = lo + m2;
-    hi += lo2 < m2;
-    return redc(hi, lo2, q, qinv_neg);
+    for (int j = 0; j < ND; ++j) acc.mac(dg[j * dstride], load_stream(kr + j * kstride));
   } else {
-    Acc128 acc;
-    if (ND > 0) {
-#pragma unroll
-      for (int j = 0; j < ND; ++j) acc.mac(dg[j * dstride], load_stream(kr + j * kstride));
-    } else {
-      for (uint32_t j = 0; j < nd_rt; ++j) acc.mac(dg[j * dstride], load_stream(kr + j * kstride));
-    }
-    return redc(acc.hi, acc.lo, q, qinv_neg);
+    for (uint32_t j = 0; j < nd_rt; ++j) acc.mac(dg[j * dstride], load_stream(kr + j * kstride));
   }
+  return redc(acc.hi, acc.lo, q, qinv_neg);
 }
 
-// key_dot for positions s and s + 1 (s even, operands 16-byte aligned) with
-// 16-byte loads, in the SPLIT form only (every modulus below 2^60, 1..7
-// digits): half the load instructions of two key_dot calls.  key_fetch2
-// issues the loads, key_comb2 forms the two sums.
-template <int ND>
-__device__ __forceinline__ void key_fetch2(const uint64_t* dg, size_t dstride, const uint64_t* kr,
-                                           size_t kstride, ulonglong2* d, ulonglong2* k) {
-  static_assert(ND > 0 && ND <= 7, "split key products");
-#pragma unroll
-  for (int j = 0; j < ND; ++j) {
-    d[j] = *reinterpret_cast<const ulonglong2*>(dg + j * dstride);
-    k[j] = load_stream2(kr + j * kstride);
-  }
-}
-template <int ND>
-__device__ __forceinline__ void key_comb2(const ulonglong2* d, const ulonglong2* k, uint64_t q,
-                                          uint64_t qinv_neg, uint64_t& t0, uint64_t& t1) {
-  constexpr uint32_t M30 = (1u << 30) - 1;
-  uint64_t a0[2] = {0, 0}, a1[2] = {0, 0}, a2[2] = {0, 0};
-#pragma unroll
-  for (int j = 0; j < ND; ++j) {
-    const uint64_t dd[2] = {d[j].x, d[j].y}, kk[2] = {k[j].x, k[j].y};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t dl = (uint32_t)dd[h] & M30, dh = (uint32_t)(dd[h] >> 30);
-      const uint32_t kl = (uint32_t)kk[h] & M30, kh = (uint32_t)(kk[h] >> 30);
-      a0[h] += (uint64_t)dl * kl;
-      a1[h] += (uint64_t)dl * kh;
-      a1[h] += (uint64_t)dh * kl;
-      a2[h] += (uint64_t)dh * kh;
-    }
-  }
-  uint64_t t[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const uint64_t m1 = a1[h] << 30, m2 = a2[h] << 60;
-    const uint64_t lo = a0[h] + m1;
-    uint64_t hi = (a1[h] >> 34) + (a2[h] >> 4) + (lo < m1);
-    const uint64_t lo2 = lo + m2;
-    hi += lo2 < m2;
-    t[h] = redc(hi, lo2, q, qinv_neg);
-  }
-  t0 = t[0];
-  t1 = t[1];
-}
-
-// key_comb2 with the reduction left lazy: redc_lazy, each sum in (0, 2q)
-// (T < nd q^2 keeps T's high word below q for nd q < 2^64).
+// The sums of two adjacent positions, every modulus below 2^60 and 1 .. 7
+// digits: operands split at bit 30 and accumulated carry-free in three 64-bit
+// sums with v_mad_u64_u32, T = a0 + a1 2^30 + a2 2^60.  The reduction is left
+// lazy, each sum in (0, 2q) (T < nd q^2 keeps T's high word below q for nd q <
+// 2^64).
 template <int ND>
 __device__ __forceinline__ void key_comb2_lazy(const ulonglong2* d, const ulonglong2* k,
                                                uint64_t q, uint64_t qinv, uint64_t& t0,
                                                uint64_t& t1) {
+  static_assert(ND > 0 && ND <= 7, "split key products");
   constexpr uint32_t M30 = (1u << 30) - 1;
   uint64_t a0[2] = {0, 0}, a1[2] = {0, 0}, a2[2] = {0, 0};
 #pragma unroll
@@ -146,46 +81,18 @@ __device__ __forceinline__ void key_comb2_lazy(const ulonglong2* d, const ulongl
 // ModDown epilogue (see ModDownEpi): the value at evaluation slot s goes to
 // slot d(s) of the output, d being the inverse Galois permutation.  ND > 0
 // fixes the digit count at compile time (ND = 0: e.nd at run time).
-template <int ND, bool SPLIT = false>
+template <int ND>
 struct EpiStore {
   static constexpr bool kPre = true;
-  static constexpr bool kPair = SPLIT && ND > 0 && ND <= 7;
   const ModDownEpi& e;
   uint32_t n, log_n;
-  // pre() for positions s and s + 1 (s even), kPair only.  The addend is
-  // loaded with the key operands; without one the first digit's words are
-  // read again (a cache hit) so that the load needs no branch.
-  struct Ops2 {
-    ulonglong2 d[kPair ? ND : 1], k[kPair ? ND : 1], add;
-  };
-  __device__ __forceinline__ void fetch2(size_t s, Ops2& o) const {
-    if constexpr (kPair) {
-      const uint32_t p = blockIdx.y, r = p >> 1, b = p & 1, i = blockIdx.z;
-      const uint64_t* dg = e.digits[r] + (size_t)i * n + s;
-      key_fetch2<ND>(dg, (size_t)e.ne * n, e.key[r] + (size_t)b * e.kl + (size_t)i * n + s,
-                     2 * e.kl, o.d, o.k);
-      const uint64_t* add = e.add[r][b];
-      o.add = *reinterpret_cast<const ulonglong2*>(add ? add + (size_t)i * n + s : dg);
-    }
-  }
-  __device__ __forceinline__ void comb2(const Ops2& o, uint64_t q, uint64_t& t0,
-                                        uint64_t& t1) const {
-    if constexpr (kPair) {
-      const uint32_t p = blockIdx.y, r = p >> 1, b = p & 1, i = blockIdx.z;
-      key_comb2<ND>(o.d, o.k, q, e.mc[i].qinv_neg, t0, t1);
-      if (e.add[r][b]) {
-        t0 = add_mod(t0, o.add.x, q);
-        t1 = add_mod(t1, o.add.y, q);
-      }
-    }
-  }
   // Q-limb key inner product plus the addend at position s.
   __device__ __forceinline__ uint64_t pre(size_t s, uint64_t q) const {
     const uint32_t p = blockIdx.y, r = p >> 1, b = p & 1, i = blockIdx.z;
     const uint64_t* dg = e.digits[r] + (size_t)i * n + s;
     const uint64_t* kr = e.key[r] + (size_t)b * e.kl + (size_t)i * n + s;
     const size_t dstride = (size_t)e.ne * n, kstride = 2 * e.kl;
-    uint64_t t = key_dot<ND, SPLIT>(dg, dstride, kr, kstride, e.nd, q, e.mc[i].qinv_neg);
+    uint64_t t = key_dot<ND>(dg, dstride, kr, kstride, e.nd, q, e.mc[i].qinv_neg);
     const uint64_t* add = e.add[r][b];
     if (add) t = add_mod(t, add[(size_t)i * n + s], q);
     return t;
@@ -208,10 +115,9 @@ struct EpiStore {
 
 // P-limb key inner product as the input of ModDown's inverse NTT: launch
 // poly p is key switch r = p / 2, component b = p % 2, limb t is P limb t.
-template <int ND, bool SPLIT = false>
+template <int ND>
 struct KskLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = SPLIT && ND > 0 && ND <= 7;
   const ModDownEpi& e;
   uint32_t n;
   __device__ __forceinline__ uint64_t get(size_t s, uint64_t q) const {
@@ -219,25 +125,24 @@ struct KskLoad {
     const uint64_t* dg = e.digits[r] + (size_t)(e.nq + t) * n + s;
     const uint64_t* kr = e.key[r] + (size_t)b * e.kl + (size_t)(e.L + t) * n + s;
     const size_t dstride = (size_t)e.ne * n, kstride = 2 * e.kl;
-    return key_dot<ND, SPLIT>(dg, dstride, kr, kstride, e.nd, q, e.mc[e.L + t].qinv_neg);
-  }
-  // get() for positions s and s + 1 (s even), kPair only.
-  struct Ops2 {
-    ulonglong2 d[kPair ? ND : 1], k[kPair ? ND : 1];
-  };
-  __device__ __forceinline__ void fetch2(size_t s, Ops2& o) const {
-    if constexpr (kPair) {
-      const uint32_t p = blockIdx.y, r = p >> 1, b = p & 1, t = blockIdx.z;
-      key_fetch2<ND>(e.digits[r] + (size_t)(e.nq + t) * n + s, (size_t)e.ne * n,
-                     e.key[r] + (size_t)b * e.kl + (size_t)(e.L + t) * n + s, 2 * e.kl, o.d,
-                     o.k);
-    }
-  }
-  __device__ __forceinline__ void comb2(const Ops2& o, uint64_t q, uint64_t& v0,
-                                        uint64_t& v1) const {
-    if constexpr (kPair) key_comb2<ND>(o.d, o.k, q, e.mc[e.L + blockIdx.z].qinv_neg, v0, v1);
+    return key_dot<ND>(dg, dstride, kr, kstride, e.nd, q, e.mc[e.L + t].qinv_neg);
   }
 };
+
+// f(ND): the digit counts with kernels of their own when FIXED, 0 (run time)
+// for the others.
+template <bool FIXED, class F>
+void with_digits(uint32_t nd, F&& f) {
+  if constexpr (FIXED) {
+    switch (nd) {
+      case 1: f(std::integral_constant<int, 1>{}); return;
+      case 2: f(std::integral_constant<int, 2>{}); return;
+      case 3: f(std::integral_constant<int, 3>{}); return;
+      default: break;
+    }
+  }
+  f(std::integral_constant<int, 0>{});
+}
 
 }  // namespace
 }  // namespace fhe

@@ -13,9 +13,9 @@ __global__ void __launch_bounds__(256)
     ntt_pass_ksk(uint64_t* __restrict__ data, size_t poly_stride, const ModConst* __restrict__ mc,
                  const uint64_t* __restrict__ tw_all, uint32_t log_n, uint32_t s_other,
                  const ModDownEpi epi) {
-  ntt_body<LIM, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, KskLoad<ND, BLK>, LimbMap, false,
-           BLK>(data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), s_other,
-                PlainStore{}, KskLoad<ND, BLK>{epi, 1u << log_n});
+  ntt_body<LIM, S, BLOCKS, true, RHO_EPILOGUE, PlainStore, KskLoad<ND>, LimbMap, false, BLK>(
+      data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(epi.L), s_other, PlainStore{},
+      KskLoad<ND>{epi, 1u << log_n});
 }
 
 // BLK: pass of the fused ModDown (moduli below 2^60), y read from the
@@ -25,9 +25,9 @@ __global__ void __launch_bounds__(256)
     ntt_pass_moddown(uint64_t* __restrict__ data, size_t poly_stride,
                      const ModConst* __restrict__ mc, const uint64_t* __restrict__ tw_all,
                      uint32_t log_n, uint32_t s_other, const ModDownEpi epi) {
-  ntt_body<LIM, S, BLOCKS, false, RHO_EPILOGUE, EpiStore<ND, BLK>, PlainLoad, LimbMap, BLK>(
+  ntt_body<LIM, S, BLOCKS, false, RHO_EPILOGUE, EpiStore<ND>, PlainLoad, LimbMap, BLK>(
       data, poly_stride, mc, tw_all, log_n, LimbMap::contiguous(0), s_other,
-      EpiStore<ND, BLK>{epi, 1u << log_n, log_n});
+      EpiStore<ND>{epi, 1u << log_n, log_n});
 }
 
 // Last forward pass of a batched ModDown over the blocked y, both polys of
@@ -324,7 +324,7 @@ __global__ void __launch_bounds__(512)
 // products of both polys at the same positions, the digits' words read
 // once, runs the first S2 inverse stages of both polys with shared
 // twiddles, and the workgroup stores its rows (one blocked group) to the
-// blocked layout.  The values stay in [0, 4q); N^-1 is applied later.
+// blocked layout, below 8q; N^-1 is applied later.
 // Up to three digits it fits 64 VGPRs without spills, so four 8-wave
 // workgroups share a CU (LDS allows four; measured 2% faster than three at
 // N=2^16, 24 limbs).
@@ -461,6 +461,17 @@ __global__ void __launch_bounds__(512)
                             blockIdx.z, lds);
 }
 
+// f(LIM): the blocked form belongs to the fused ModDown, whose moduli all suit
+// the wide lazy range.
+template <bool BLK, class F>
+void with_pass_lim(const Context& c, F&& f) {
+  if constexpr (BLK)
+    f(std::integral_constant<int, 16>{});
+  else
+    with_lim(c, f);
+}
+
+// npoly is even: polys 2 r and 2 r + 1 belong to key switch r.
 template <int S, bool BLK = false>
 void launch_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq, uint32_t s_other,
                     const ModDownEpi& epi) {
@@ -470,50 +481,31 @@ void launch_moddown(Context& c, uint64_t* y, uint32_t npoly, uint32_t nq, uint32
   if constexpr (BLK) {
     // Both polys of each key switch in one workgroup (blocked y, digits
     // 1..7): rows per workgroup = one blocked group.
-    constexpr uint32_t pair_lines = 512u >> (S - 2);
-    if (npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
-      const dim3 grid((1u << s_other) / pair_lines, npoly / 2, nq);
+    const dim3 grid((1u << s_other) / pair_lines<S>(), npoly / 2, nq);
 #define CASE(D, RAW)                                                                         \
   case D:                                                                                    \
     FHE_LAUNCH(c, name, (ntt_pass_moddown_pair<S, D, RAW>), grid, dim3(512), 0, y, c.d_const, \
                c.d_tw_fwd, c.log_n, s_other, epi);                                           \
     return;
-      if (epi.raw) {
-        switch (epi.nd) {
-          CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
-        }
-      } else {
-        switch (epi.nd) {
-          CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
-          CASE(6, false) CASE(7, false)
-        }
+    if (epi.raw) {
+      switch (epi.nd) {
+        CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
       }
-#undef CASE
+    } else {
+      switch (epi.nd) {
+        CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
+        CASE(6, false) CASE(7, false)
+      }
     }
+#undef CASE
   }
-  // The blocked form belongs to the fused ModDown, whose moduli all suit the
-  // wide lazy range.
-  auto launch = [&](auto nd) {
-    auto go = [&](auto lim) {
+  with_digits<!BLK>(epi.nd, [&](auto nd) {  // blocked: eight digits
+    with_pass_lim<BLK>(c, [&](auto lim) {
       FHE_LAUNCH(c, name, (ntt_pass_moddown<decltype(lim)::value, S, decltype(nd)::value, BLK>),
                  dim3(tiles, npoly, nq), dim3(256), 0, y, (size_t)nq * c.n, c.d_const,
                  c.d_tw_fwd, c.log_n, s_other, epi);
-    };
-    if constexpr (BLK)
-      go(std::integral_constant<int, 16>{});
-    else
-      with_lim(c, go);
-  };
-  switch (epi.nd) {
-#define CASE(D)                                                                               \
-  case D:                                                                                     \
-    launch(std::integral_constant<int, D>{});                                                 \
-    return;
-    CASE(1) CASE(2) CASE(3)
-#undef CASE
-    default:
-      launch(std::integral_constant<int, 0>{});
-  }
+    });
+  });
 }
 
 template <int S, bool BLK = false>
@@ -522,55 +514,35 @@ void launch_ksk(Context& c, uint64_t* ext, uint32_t npoly, uint32_t s_other,
   using G = Geo<S, RHO_EPILOGUE>;
   const uint32_t tiles = (1u << s_other) / (256 / G::TPL);
   const char* name = "ntt_inv_blocks_ksk";
-  const dim3 grid(tiles, npoly, c.K);
   const size_t ps = (size_t)c.K * c.n;
   if constexpr (BLK) {
     // Both polys of each key switch in one workgroup (blocked output, digits
     // 1..7, no final scaling): rows per workgroup = one blocked group.
-    constexpr uint32_t pair_lines = 512u >> (S - 2);
-    if (npoly % 2 == 0 && epi.nd >= 1 && epi.nd <= 7) {
-      const dim3 pgrid((1u << s_other) / pair_lines, npoly / 2, c.K);
+    const dim3 grid((1u << s_other) / pair_lines<S>(), npoly / 2, c.K);
 #define CASE(D, RAW)                                                                        \
   case D:                                                                                   \
-    FHE_LAUNCH(c, name, (ntt_pass_ksk_pair<S, D, RAW>), pgrid, dim3(512), 0, ext, ps,       \
+    FHE_LAUNCH(c, name, (ntt_pass_ksk_pair<S, D, RAW>), grid, dim3(512), 0, ext, ps,        \
                c.d_const, c.d_tw_inv, c.d_tw_fwd, c.log_n, s_other, epi);                   \
     return;
-      if (epi.raw) {
-        switch (epi.nd) {
-          CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
-        }
-      } else {
-        switch (epi.nd) {
-          CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
-          CASE(6, false) CASE(7, false)
-        }
+    if (epi.raw) {
+      switch (epi.nd) {
+        CASE(1, true) CASE(2, true) CASE(3, true) CASE(4, true)
       }
-#undef CASE
+    } else {
+      switch (epi.nd) {
+        CASE(1, false) CASE(2, false) CASE(3, false) CASE(4, false) CASE(5, false)
+        CASE(6, false) CASE(7, false)
+      }
     }
-  }
-  // The blocked form belongs to the fused ModDown, whose moduli all suit the
-  // wide lazy range.
-  auto launch = [&](auto nd) {
-    auto go = [&](auto lim) {
-      FHE_LAUNCH(c, name, (ntt_pass_ksk<decltype(lim)::value, S, decltype(nd)::value, BLK>),
-                 grid, dim3(256), 0, ext, ps, c.d_const, c.d_tw_inv, c.log_n, s_other,
-                 epi);
-    };
-    if constexpr (BLK)
-      go(std::integral_constant<int, 16>{});
-    else
-      with_lim(c, go);
-  };
-  switch (epi.nd) {
-#define CASE(D)                                                                         \
-  case D:                                                                               \
-    launch(std::integral_constant<int, D>{});                                           \
-    return;
-    CASE(1) CASE(2) CASE(3)
 #undef CASE
-    default:
-      launch(std::integral_constant<int, 0>{});
   }
+  with_digits<!BLK>(epi.nd, [&](auto nd) {  // blocked: eight digits
+    with_pass_lim<BLK>(c, [&](auto lim) {
+      FHE_LAUNCH(c, name, (ntt_pass_ksk<decltype(lim)::value, S, decltype(nd)::value, BLK>),
+                 dim3(tiles, npoly, c.K), dim3(256), 0, ext, ps, c.d_const, c.d_tw_inv, c.log_n,
+                 s_other, epi);
+    });
+  });
 }
 
 }  // namespace
@@ -586,7 +558,8 @@ void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uin
   if (npoly == 0) return;
   if (npoly > 2 * MAX_KS_BATCH) throw ArgError("ModDown batch too large");
   if (!moddown_fused_ok(c, nq)) throw ArgError("fused ModDown does not apply");
-  if (epi.raw && (epi.nd > RAW_MAX_DIGITS || npoly % 2))
+  if (npoly % 2) throw ArgError("ModDown takes both polys of each key switch");
+  if (epi.raw && epi.nd > RAW_MAX_DIGITS)
     throw ArgError("digits without their last pass do not apply");
   const uint32_t s1 = (c.log_n + 1) / 2;
   switch (c.log_n) {

@@ -12,7 +12,6 @@ namespace {
 // kernel of 112 us to write them and a first pass of 153, now 111 in all.
 struct SignedLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   const int64_t* coef;
   const ModConst* mc;
   uint32_t n, mod0;
@@ -22,22 +21,15 @@ struct SignedLoad {
     const uint64_t r = a - mulhi64(a, mc[mod0 + blockIdx.z].mu64) * q;
     return x < 0 ? 2 * q - r : r;
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
 };
 // Input of an inverse transform of one poly, read from another buffer.
 struct FromLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   const uint64_t* src;
   uint32_t n;
   __device__ __forceinline__ uint64_t get(size_t g, uint64_t) const {
     return src[(size_t)blockIdx.z * n + g];
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
 };
 
 template <int LIM, int S, int KIND, bool INV, class Map, class Load>

@@ -85,17 +85,9 @@ __device__ __forceinline__ uint64_t* poly_base(const TableMap& m, uint64_t*, siz
 // Final stores go through `store.fin(base, offset_in_limb, value, t, q)`,
 // with t = store.pre(offset_in_limb, q) when Store::kPre.
 // The first pass's input comes from `load.get(offset_in_limb, q)` instead
-// of data when Load::kLoad.  kPair functors also produce the terms of two
-// adjacent positions from 16-byte loads in two steps, fetch2 (every load of
-// the pair, issued together into an Ops2) and comb2 (the arithmetic).
-// Prefetching the next pair's operands before a pair's products was
-// measured slower: the extra registers cost more waves than they hide.
+// of data when Load::kLoad.
 struct PlainLoad {
   static constexpr bool kLoad = false;
-  static constexpr bool kPair = false;
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
   __device__ __forceinline__ uint64_t get(size_t, uint64_t) const { return 0; }
 };
 
@@ -241,8 +233,8 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
   static_assert(!WL || G::TPL <= 64, "a block line spans one wavefront");
   // Staged position k of this thread: per wavefront (WL) or per workgroup.
   // PAIR (every BLOCKS launch): a lane stages two adjacent positions at a
-  // time, so plain staged loads and stores and the kPair functors' operands
-  // are 16-byte accesses: staged position k is
+  // time, so plain staged loads and stores are 16-byte accesses: staged
+  // position k is
   // wave * 64R + (k / 2) * 128 + 2 * lane + k % 2.
   constexpr bool PAIR = WL;
   constexpr bool PLAIN_ST = std::is_same<Store, PlainStore>::value;
@@ -285,18 +277,7 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
 
     if (sp == 0 && (contiguous || BLK_IN)) {
       const size_t wg0 = ((size_t)blockIdx.x * LINES) << S;
-      if constexpr (Load::kPair && PAIR && !BLK_IN) {
-#pragma unroll
-        for (int k = 0; k < R; k += 2) {
-          const uint32_t p = staged(k);
-          typename Load::Ops2 ops;
-          uint64_t v0, v1;
-          load.fetch2(wg0 + p, ops);
-          load.comb2(ops, q, v0, v1);
-          lds[lds_idx(p >> S, p & (G::LEN - 1), G::PITCH)] = v0;
-          lds[lds_idx((p + 1) >> S, (p + 1) & (G::LEN - 1), G::PITCH)] = v1;
-        }
-      } else if constexpr (PAIR && !Load::kLoad && !BLK_IN) {
+      if constexpr (PAIR && !Load::kLoad && !BLK_IN) {
 #pragma unroll
         for (int k = 0; k < R; k += 2) {
           const uint32_t p = staged(k);
@@ -348,22 +329,13 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
     constexpr bool kFinalContig = !INV && KIND != COLS;
     if (Store::kPre && LAST && sp == (kFinalContig ? 0 : NSP - 1)) {
       const size_t wg0 = ((size_t)blockIdx.x * LINES) << S;
-      if constexpr (Store::kPair && PAIR && kFinalContig) {
 #pragma unroll
-        for (int k = 0; k < R; k += 2) {
-          typename Store::Ops2 ops;
-          store.fetch2(wg0 + staged(k), ops);
-          store.comb2(ops, q, pre[k], pre[k + 1]);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-          const uint32_t u = thi | ((uint32_t)k << w) | tlo;
-          const size_t g = kFinalContig ? wg0 + staged(k)
-                           : KIND == COLS ? gline + ((size_t)u << s_other)
-                                          : ((size_t)gline << S) + u;
-          pre[Store::kPre ? k : 0] = store.pre(g, q);
-        }
+      for (int k = 0; k < R; ++k) {
+        const uint32_t u = thi | ((uint32_t)k << w) | tlo;
+        const size_t g = kFinalContig ? wg0 + staged(k)
+                         : KIND == COLS ? gline + ((size_t)u << s_other)
+                                        : ((size_t)gline << S) + u;
+        pre[Store::kPre ? k : 0] = store.pre(g, q);
       }
     }
 
@@ -474,10 +446,6 @@ __device__ __forceinline__ void ntt_body(uint64_t* __restrict__ data, size_t pol
 // butterflies; fin then writes f(y, t).
 struct PlainStore {
   static constexpr bool kPre = false;
-  static constexpr bool kPair = false;
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
   __device__ __forceinline__ uint64_t pre(size_t, uint64_t) const { return 0; }
   __device__ __forceinline__ void fin(uint64_t* base, size_t g, uint64_t v, uint64_t,
                                       uint64_t) const {
@@ -528,7 +496,6 @@ constexpr int MODUP_MAX_CT = 32;
 template <bool KEEP>
 struct SrcLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   const uint64_t* const* src;  // MODUP_MAX_CT entries in kernel arguments
   uint32_t n;
   uint64_t* digits;
@@ -539,9 +506,6 @@ struct SrcLoad {
     if (KEEP) digits[(((size_t)ct * nd + i / alpha) * ne + i) * n + g] = v;
     return v;
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
 };
 struct SrcPtrs {
   const uint64_t* p[MODUP_MAX_CT];

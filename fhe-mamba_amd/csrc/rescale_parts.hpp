@@ -18,7 +18,6 @@ struct RescalePtrs {
 };
 struct LastLimbLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   const uint64_t* const* a;  // RESCALE_MAX entries in kernel arguments
   uint32_t npoly;
   size_t poly_words, last_off;
@@ -26,13 +25,9 @@ struct LastLimbLoad {
     const uint32_t y = blockIdx.y;
     return a[y / npoly][(size_t)(y % npoly) * poly_words + last_off + g];
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
 };
 struct LiftLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   const uint64_t* last;  // [npoly][N], coefficient form mod q_l, in [0, q_l)
   const ModConst* mc;
   const uint64_t* rs;
@@ -44,13 +39,9 @@ struct LiftLoad {
     const uint64_t r = reduce_2q(x - mulhi64(x, mc[i].mu64) * q, q);
     return x > half ? sub_mod(r, rs[((size_t)l * L + i) * 4], q) : r;
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
 };
 struct RescaleStore {
   static constexpr bool kPre = true;
-  static constexpr bool kPair = false;
   const uint64_t* const* a;  // RESCALE_MAX entries in kernel arguments
   uint64_t* const* out;
   const uint64_t* rs;
@@ -59,9 +50,6 @@ struct RescaleStore {
     const uint32_t y = blockIdx.y;
     return a[y / npoly][((size_t)(y % npoly) * (l + 1) + blockIdx.z) * n + s];
   }
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
   __device__ __forceinline__ void fin(uint64_t*, size_t s, uint64_t y, uint64_t x,
                                       uint64_t q) const {
     const uint32_t i = blockIdx.z, p = blockIdx.y;

@@ -32,13 +32,9 @@ struct SmallConv {
 };
 struct ConvLoad {
   static constexpr bool kLoad = true;
-  static constexpr bool kPair = false;
   static constexpr bool kBulk = true;
   const SmallConv& a;
   uint32_t mod;
-  struct Ops2 {};
-  __device__ __forceinline__ void fetch2(size_t, Ops2&) const {}
-  __device__ __forceinline__ void comb2(const Ops2&, uint64_t, uint64_t&, uint64_t&) const {}
   __device__ __forceinline__ uint64_t get(size_t, uint64_t) const { return 0; }
   template <int R>
   __device__ __forceinline__ void bulk(const size_t (&g)[R], uint64_t (&x)[R]) const {
@@ -151,19 +147,6 @@ void with_ring(const Context& c, F&& f) {
     default: throw ArgError("unsupported ring dimension");
   }
 }
-template <bool FIXED, class F>
-void with_digits(uint32_t nd, F&& f) {
-  if constexpr (FIXED) {
-    switch (nd) {
-      case 1: f(std::integral_constant<int, 1>{}); return;
-      case 2: f(std::integral_constant<int, 2>{}); return;
-      case 3: f(std::integral_constant<int, 3>{}); return;
-      default: break;
-    }
-  }
-  f(std::integral_constant<int, 0>{});
-}
-
 SmallPlan small_plan(const ConvPlan& pl, uint32_t src_limb, uint32_t src_mod) {
   return SmallPlan{pl.d_qhat_inv, pl.d_qhat_mont, pl.nsrc, pl.ndst, src_limb, src_mod};
 }
