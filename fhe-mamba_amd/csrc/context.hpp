@@ -395,7 +395,7 @@ void moddown_mid(Context& c, const uint64_t* ext_p, uint64_t* y, uint32_t npoly,
 void moddown_fused(Context& c, uint64_t* ext_p, uint64_t* y, uint32_t npoly, uint32_t nq,
                    const ConvPlan& pl, const ModDownEpi& epi);
 // Rescale of [npoly][nq][N] into out [npoly][nq-1][N] (out != a) in three
-// launches, or four (rescale.hip has the rule), for ring dimensions 2^13..2^17.
+// launches, or four (rescale_by_columns and its moduli rule), for ring dimensions 2^13..2^17.
 void rescale_fused(Context& c, uint64_t* out, const uint64_t* a, uint32_t npoly, uint32_t nq);
 // The same for `count` inputs as[r] into outs[r] (each [npoly][nq][N] into
 // [npoly][nq-1][N], no output aliasing any input): up to 16 inputs share

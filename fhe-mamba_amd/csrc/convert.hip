@@ -54,8 +54,8 @@ __global__ void __launch_bounds__(256)
 // gives the eight sums of four targets (32 rows) at 32 column rows (32
 // columns) from four sources a step.  One 32-bit Montgomery step of the about
 // 75-bit T_k, T_k + m t_k = 2^32 r, leaves r = sum_i v_i c_ik in (0, 3 t_k)
-// after adding t_k.  Per output that is about 17 VALU instructions whatever
-// the number of sources, where 64-bit multiply-adds took 4 a source and 25.
+// after adding t_k.  Per output that is 19 VALU instructions whatever the number
+// of sources, where 64-bit multiply-adds took 4 a source and 25.
 constexpr uint32_t MAX_CONV_SRC = 16;
 
 // What one (poly, column) tile converts.  Poly p of the launch uses plan
@@ -75,8 +75,8 @@ struct MidPlan {
   uint32_t nsrc, ndst, src_mod0, src_limb0, skip_at, skip_len, qlimbs;
 };
 struct MidArgs {
-  const uint64_t* src;        // blocked, inverse block stages done, [0, 4q)
-  uint64_t* out;              // blocked, forward column stages done, [0, 8q)
+  const uint64_t* src;        // blocked, inverse block stages done, below 8q
+  uint64_t* out;              // blocked, forward column stages done, below 12q
   size_t src_group_words, out_group_words;
   MidPlan plan[MID_MAXPLAN];
   uint32_t nplan, L;

@@ -39,8 +39,9 @@ def test_keyswitch_every_level(setup):
 
 
 def test_rescale_shapes(setup):
-    """Rescale (four-launch form at these ring dimensions) of 1 and 2 polys
-    at every level, against the oracle."""
+    """Rescale (the column kernel's smallest workgroups, or four launches where
+    q_l is too large for it) of 1 and 2 polys at every level, against the
+    oracle."""
     ctx, orc, s = setup
     rng = np.random.default_rng(11)
     for npoly in (1, 2):
@@ -82,9 +83,9 @@ def test_hoisted_rotations(setup):
 
 
 def test_benchmark_shape_rotations():
-    """Eight hoisted rotations (16 polys x 256 columns: the 4-wave middle
-    kernel) and one single rotation one level down (the 8-wave one) at the
-    benchmark's parameters."""
+    """Eight hoisted rotations (16 polys x 256 columns, several rounds of
+    workgroups) and one single rotation one level down (one round, 23 targets)
+    at the benchmark's parameters."""
     q, p = O.gen_moduli(16, 23, 59, 60, 3)
     ctx, orc = F.Context(16, q, p, 3, sampling="seeded"), O.Ctx(16, q, p, 3)
     assert (ctx.L, ctx.K) == (24, 8)
@@ -167,8 +168,8 @@ def test_many_digits(log_n, depth, dnum):
 
 
 def test_full_batch_small_ring():
-    """32 hoisted rotations at N=2^13 (64 polys x 64 columns: the 4-wave
-    middle kernel with two column lines per wavefront)."""
+    """32 hoisted rotations at N=2^13 (64 polys x 64 columns, 8 targets: the
+    4-wave middle kernel, two column lines per wavefront, one target batch)."""
     q, p = O.gen_moduli(13, 7, 50, 60, 2)
     ctx, orc = F.Context(13, q, p, 2, sampling="seeded"), O.Ctx(13, q, p, 2)
     s = orc.secret(8)
@@ -187,8 +188,9 @@ def test_classical128_chain_key_switch():
     """The reference's audited classical-128 chain (N=2^17, 45 Q + 12 P
     primes, four digits: the golden OpenFHE chain) at the full level and at
     31 limbs: relinearisation key switch and hoisted rotations, word for
-    word against the oracle (the fused middle kernel holds the 12 source
-    lines of a column in up to 160 KB of LDS per workgroup)."""
+    word against the oracle (16-wave workgroups of the fused middle kernel,
+    the 12 source lines and 16 target lines of a column in 120 KB of LDS: three
+    batches of targets, the last one ragged, and two)."""
     import json
     import os
     gold = json.load(open(os.path.join(os.path.dirname(__file__), "golden",
@@ -204,8 +206,8 @@ def test_classical128_chain_key_switch():
     gal = [O.galois_elt(r, ctx.n) for r in (1, -8, 2, 4, -16, 32, 64, -128, 256)]
     gkeys = [orc.galois_key(s, g, 60 + i) for i, g in enumerate(gal)]
     dgk = [ctx.load_key(k) for k in gkeys]
-    # 2 rotations: one 16-wave middle-kernel launch; at 31 limbs also 3
-    # (8-wave) and 9 (4-wave), the 12 sources in two groups each time
+    # 12 sources are three whole four-source steps; at 31 limbs ModUp's last
+    # digit has 7, and 2, 3 and 9 rotations are 2, 3 and 9 rounds of workgroups
     for nq, counts in ((45, (2,)), (31, (2, 3, 9))):
         a = residues(rng, ctx.q[:nq], (1,), ctx.n)
         assert np.array_equal(ctx.keyswitch(ctx.upload(a), dkey).numpy(),
@@ -223,11 +225,11 @@ def test_classical128_chain_key_switch():
 
 def test_decode_chain_conversion_groups():
     """The decode's N=2^16 chain (45 Q + 15 P primes, dnum 3), whose
-    conversions have 15 sources (two groups of at most eight), word for word
-    against the oracle in each middle-kernel launch shape: a relinearisation
-    key switch (one ciphertext: 16-wave workgroups), 3 hoisted rotations
-    (8-wave) and 9 (4-wave), at 45 limbs and at 20 (ModUp digits of 15 and 5
-    sources)."""
+    conversions have 15 sources (four four-source steps, the last of three),
+    word for word against the oracle: a relinearisation key switch (one round of
+    8-wave workgroups), 3 hoisted rotations (two rounds) and 9 (six), at 45 limbs
+    (target batches of 8, the last one ragged) and at 20 (ModUp digits of 15
+    and 5 sources)."""
     q, p = O.gen_moduli(16, 44, 59, 60, 3)
     print(f"[decode chain] N=2^16 Q={len(q)} P={len(p)} dnum=3", flush=True)
     ctx, orc = F.Context(16, q, p, 3, sampling="seeded"), O.Ctx(16, q, p, 3)
