@@ -45,15 +45,15 @@ HBM_PEAK = 8.0e12  # B/s, MI355X HBM3E
 # hash of the kernel sources they were measured on.  A build from other
 # sources reports traffic as null.
 MEASURED_TRAFFIC = {
-    "csrc_sha16": "4c733eb8566fbd52",
+    "csrc_sha16": "0be806f9931d846c",
     "kernels": {
         # 30-rotation batch launches of the rotation step
-        "ntt_fwd_blocks_moddown": 3_097_606_758 + 754_974_720,
-        "k_moddown_mid": 253_034_906 + 754_984_243,
-        "ntt_inv_blocks_ksk": 776_276_992 + 251_658_240,
+        "ntt_fwd_blocks_moddown": 3_097_693_056 + 754_974_720,
+        "k_moddown_mid": 253_034_214 + 754_988_160,
+        "ntt_inv_blocks_ksk": 776_266_291 + 251_658_240,
         # NTT batch (64 ciphertexts x 2 polys x 24 limbs): one pass, and the MAC
-        "ntt_pass": 1_636_242_637 + 1_610_612_736,
-        "k_mac": 2_416_047_514 + 25_165_824,
+        "ntt_pass": 1_636_308_019 + 1_610_612_736,
+        "k_mac": 2_416_047_718 + 25_165_824,
     },
 }
 
