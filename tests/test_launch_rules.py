@@ -99,7 +99,8 @@ def test_rescale_route(rules):
         assert columns == (s1 > 7 or tiles <= 1024 or tiles * l <= 32 * 1024), what
         assert nw in (2, 4, 8, 16) and (nw == 2 or l > nw // 2 * lines_per_wave(s1)), what
         assert nw < 16 or (tiles <= 512 and s1 < 9), what
-    want = {(7, 4096, 1): 2, (9, 4096, 1): 2, (8, 8192, 4): 4, (8, 512, 29): 16, (7, 128, 44): 16, (9, 512, 44): 8,
+    want = {(7, 4096, 1): 2, (9, 4096, 1): 2, (8, 8192, 4): 4, (8, 512, 29): 16,
+            (7, 128, 44): 16, (9, 512, 44): 8,
             (8, 768, 29): 8, (7, 1024, 44): 8, (7, 1280, 19): 4, (8, 8192, 44): 8}
     got = rules("rescale", [(*s, 0, 0) for s in want])
     assert {s: r[1] for s, r in zip(want, got)} == want
